@@ -1,9 +1,12 @@
 // The ears on the device (imi/core/ears.{h,cpp}): 16 kHz samples -> [positions][n_out] rows for the brain's
 // prefill. Kernel arguments and launchers.
 //
-// Layouts: float tables as [cols / 8][rows_pad][8] (F16 bits or F32; element (r, k) at ((k / 8) rows_pad + r) 8 +
-// k % 8, so a wave's 64 rows read 1 KB per 8 columns); table inputs feature-major [cols][ldx] (positions contiguous,
-// ldx a multiple of 4); the residual stream and the layer's q|k|v or b|c|x rows position-major [P][width].
+// Layouts: float tables (F16 bits or F32) in tiles of 32 columns x 16 rows, [cols / 32][rows_pad / 16], columns and rows
+// padded with zeros. A tile holds the 8 weights of each lane of the 16 x 16 x 4 products: lane 16 (k % 4) + r % 16, value
+// k % 32 / 4; F16 as [64][8], F32 as [2][64][4] (values 0-3, then 4-7). Table inputs likewise, [cols / 32][ldx / 16] tiles
+// of [2][64][4] floats with positions in the place of rows (ldx a multiple of 16; features padded to a multiple of 32, the
+// padding's contents unused). Images and powers feature-major [features][ld]; the residual stream and the layer's q|k|v or
+// b|c|x rows position-major [P][width].
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -11,7 +14,6 @@
 
 namespace sh {
 
-constexpr int EA_NP = 4;          // positions per table thread (wave-uniform)
 constexpr int EA_MAX_WIN = 64;    // attention window the kernel takes (one lane per key)
 constexpr int EA_MAX_D = 128;
 
@@ -30,18 +32,25 @@ struct etab {
     bool f32 = false;
 };
 
+enum ea_out : int {
+    EO_POS = 0,     // position-major [P][ldo]
+    EO_FEAT = 1,    // feature-major [rows'][ldo]
+    EO_TABLE = 2,   // a table's input (ldo positions)
+};
+
 struct etab_args {
     etab W;
-    const float* x;     // [cols][ldx]
-    int ldx, P;         // P: positions computed and stored (ldx >= P rounded up to 4)
+    const float* x;     // a table's input, [cols][ldx]
+    int ldx, P;         // P: positions computed and stored (ldx >= P rounded up to 16)
     const float* bias;  // [rows] or null
     float* out;
     int ldo;
-    bool xt_out;        // out feature-major [rows'][ldo] (else position-major [P][ldo])
+    int out_kind;       // ea_out
 };
 
 hipError_t launch_etab(int epi, const etab_args& a, hipStream_t s);
 
+// (fx, a1, xf, h and act below are table inputs, written in that layout)
 // fx[k][fr] = hann[k] * pcm[fr * hop + k] (0 past the clip or past n_fr), k < n_fft, fr < ldf
 hipError_t launch_eframes(const float* pcm, int n, const float* hann, int n_fft, int hop, int n_fr, float* fx, int ldf,
                           hipStream_t s);
@@ -52,7 +61,7 @@ hipError_t launch_emel(const float* pw, int ldp, const float* fb, const int2* sp
 // first stride-2 3x3 conv of the mel image (one input channel) + SiLU: a0[c][t][f], t < T2, f < F2
 hipError_t launch_econv0(const float* mel, int n_fr, int n_mel, const float* w9, const float* b, int C, float* a0,
                          hipStream_t s);
-// depthwise stride-2 3x3 conv: in[c][Ti][Fi] (channel stride ldi) -> out[c][To][Fo] (channel stride ldo)
+// depthwise stride-2 3x3 conv: in[c][Ti][Fi] (channel stride ldi) -> out[c][To Fo] (a table's input of ldo positions)
 hipError_t launch_edw(const float* in, int Ti, int Fi, int ldi, const float* w9, const float* b, int C, float* out,
                       int ldo, hipStream_t s);
 // xf[(c F8 + f)][p] = a[c][p F8 + f] for p < P (zero for P <= p < ldf)

@@ -39,144 +39,133 @@ __device__ __forceinline__ float rms_scale_half(const float* x, int n, float eps
 }
 
 
-// 8 columns of one row, raw: F16 bits (one 16-byte load) or F32 (two)
+// where feature e of position p sits in a table's input (sh_ears.h)
+__device__ __forceinline__ size_t xat(int e, int p, int ldx) {
+    return ((((size_t)(e >> 5) * (ldx >> 4) + (p >> 4)) * 2 + ((e >> 4) & 1)) * 64 + (e & 3) * 16 + (p & 15)) * 4 + ((e >> 2) & 3);
+}
+
+// a lane's 8 weights of a 32-column chunk, raw: F16 bits (one 16-byte load) or F32 (two)
 template <bool F32W> struct wraw;
 template <> struct wraw<false> { uint4 a; };
 template <> struct wraw<true> { float4 a, b; };
 
 template <bool F32W>
-__device__ __forceinline__ wraw<F32W> wload(const void* w, size_t at) {
+__device__ __forceinline__ wraw<F32W> wload(const void* w, size_t tile, int lane) {
     wraw<F32W> r;
     if constexpr (F32W) {
-        const float4* p = static_cast<const float4*>(w) + at * 2;
+        const float4* p = static_cast<const float4*>(w) + tile * 128 + lane;
         r.a = p[0];
-        r.b = p[1];
+        r.b = p[64];
     } else {
-        r.a = static_cast<const uint4*>(w)[at];
+        r.a = static_cast<const uint4*>(w)[tile * 64 + lane];
     }
     return r;
 }
 template <bool F32W>
-__device__ __forceinline__ void wconv(const wraw<F32W>& r, float (&o)[8]) {
+__device__ __forceinline__ float wval(const wraw<F32W>& r, int s) {   // (s known at compile time)
     if constexpr (F32W) {
-        o[0] = r.a.x; o[1] = r.a.y; o[2] = r.a.z; o[3] = r.a.w; o[4] = r.b.x; o[5] = r.b.y; o[6] = r.b.z; o[7] = r.b.w;
+        const float o[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
+        return o[s];
     } else {
         const unsigned v[4] = {r.a.x, r.a.y, r.a.z, r.a.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            o[2 * i] = h2f((uint16_t)(v[i] & 0xffffu));
-            o[2 * i + 1] = h2f((uint16_t)(v[i] >> 16));
-        }
+        return h2f((uint16_t)((v[s >> 1] >> (16 * (s & 1))) & 0xffffu));
     }
 }
 
 // The float tables on the matrix cores, in imi_wg_group12's order (imi/core/tables.cpp:522-556): one chain
-// acc = fma(w, x, acc) per row and position over the columns in order. v_mfma_f32_4x4x1_16b_f32 forms
-// d[l][i] = fma(a[4 (l / 4) + i], b[l], c[l][i]) with one rounding, bit for bit the VALU's fmaf (measured over 10^6
-// random cases with denormals, signed zeros and fused cancellation), so one instruction per column advances 16 blocks
-// of 4 rows x 4 positions of those chains by one step each, in column order. Lane l supplies its own row's weight (a)
-// and the input of position l % 4 (b); it holds rows 4 (l / 4) .. + 3 of position l % 4. A workgroup is 64 rows by
-// 4 waves x NMF position quads (NMF instructions per column and wave, one weight conversion); a wave keeps DW weight
-// loads in flight and stages its inputs position-major in LDS 128 columns at a time (one chunk ahead), 8 columns read
-// per 16-byte pair (a broadcast of the same word to every lane would cost the LDS its full return bandwidth). Every
-// global load is unconditional (indices clamped into the buffers; no product reads a column past the table, whose
-// width is a multiple of 8), so the compiler's wait counts stay exact.
-template <int EPI, bool F32W, int NMF>
+// acc = fma(w, x, acc) per row and position over the columns in order. v_mfma_f32_16x16x4_f32 runs four columns of 16
+// rows x 16 positions: its four K steps are four fused multiply-adds in order, each rounded once, bit for bit the VALU's
+// fmaf chain (measured over 3 M random cases of spread exponents). A chain then takes 8 cycles a column, the rate of one
+// matrix core in fp32, with a single chain per wave in flight; v_mfma_f32_4x4x1_16b_f32, one column per instruction,
+// is as fast only with two waves to cover its 15-cycle dependency, and wants a weight conversion and an operand word per
+// lane for every 64 x 4 outputs and column, where this takes them for 16 x 16 outputs and four columns.
+// A wave is 16 rows x 16 MP positions, a workgroup 4 waves over 64 rows. Lane l supplies row l % 16, column l / 16 of the
+// four (a) and position l % 16 of that column (b); it holds rows 4 (l / 16) .. + 3 at position l % 16. Tables and inputs
+// are laid out so that a lane's operands of 32 columns are whole 16-byte words and a wave reads 1 KB pieces (a vector
+// load costs its wave about as many cycles as one of these products), requested DC chunks of 32 columns ahead. Every
+// global load is unconditional (chunk indices clamped; past the table's last column nothing is multiplied), so the
+// compiler's wait counts stay exact.
+// At 384 positions: b|c|x 2304 x 768 33.0 -> 21.3 us, gate|up 4096 x 768 44.7 -> 30.2, down 768 x 2048 48 -> 37, the
+// 4096-wide pre_encode 90.7 -> 48.0; at 29 positions gate|up 12.6 -> 9.4, down 25 -> 16.6 (with feature-major inputs read
+// a word per step: 28.0, 44.0 and 65.3 for the first, second and fourth, 24.6 for the last). Bound by the vector loads
+// (3 KB per 32 columns and 16 x 16 outputs), then by the chains' 8 cycles a column.
+template <int EPI, bool F32W, int MP>
 __global__ __launch_bounds__(ET) void k_etab(etab_args a) {
     typedef float v4f __attribute__((ext_vector_type(4)));
-    constexpr int KC = 128, KCP = KC + 4, DW = 8, NP = 4 * NMF;
-    __shared__ __align__(16) float xs[ET / 64][2][NP][KCP];
+    constexpr int DC = MP == 4 ? 2 : MP == 2 ? 4 : 8;
     constexpr bool EXPE = EPI == EE_GLU || EPI == EE_SILU;   // epilogues that take e^x
     __shared__ uint64_t eE[ET / 64][EXPE ? 32 : 1];         // expf's table, a copy per wave (no memory round trip)
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), q = lane & 3;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), li = lane & 15, lq = lane >> 4;
+    const int nt = a.W.rows_pad / 16, tile = (int)blockIdx.x * (ET / 64) + wv, p0 = (int)blockIdx.y * 16 * MP;
+    if (tile >= nt) return;   // (whole waves; no barriers below)
     const uint64_t et = EXPE ? kExp2Tab[lane & 31] : 0;      // (requested first: its wait needs nothing later)
-    const int r = blockIdx.x * 64 + lane, p0 = (blockIdx.y * 4 + wv) * NP;
-    const int rp = a.W.rows_pad, K = a.W.cols, nk8 = K >> 3, nch = (K + KC - 1) / KC;
-    const size_t ldx = (size_t)a.ldx;
-    const int rr = r < rp ? r : rp - 1;   // lanes past the table read its last row (nothing stored)
-    float4 st[KC / 64][NMF];
-    wraw<F32W> wq[DW];
+    const int K = a.W.cols, nst = K / 4, nch = (K + 31) / 32, np = a.ldx / 16;
+    const float4* xs[MP];   // (position tiles past ldx re-read the last one)
 #pragma unroll
-    for (int i = 0; i < DW; i++) wq[i] = wload<F32W>(a.W.w, (size_t)(i < nk8 ? i : nk8 - 1) * rp + rr);
-    v4f acc[NMF];
+    for (int m = 0; m < MP; m++) xs[m] = reinterpret_cast<const float4*>(a.x) + (size_t)min(p0 / 16 + m, np - 1) * 128 + lane;
+    wraw<F32W> wr[DC];
+    float4 xr[DC][2][MP];
+    auto request = [&](int c, int d) {
+        const int cc = min(c, nch - 1);
+        wr[d] = wload<F32W>(a.W.w, (size_t)cc * nt + tile, lane);
 #pragma unroll
-    for (int m = 0; m < NMF; m++) acc[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int c = -1; c < nch; c++) {
-        // chunk c + 1's inputs are requested (clamped to the last chunk), chunk c runs from LDS, then c + 1 is stored
-        {
-            const int cn = c + 1 < nch ? c + 1 : nch - 1;
+        for (int h = 0; h < 2; h++)
 #pragma unroll
-            for (int i = 0; i < KC / 64; i++) {
-                const int k = min(cn * KC + lane + 64 * i, K - 1);
+            for (int m = 0; m < MP; m++) xr[d][h][m] = xs[m][((size_t)cc * np * 2 + h) * 64];
+    };
+    auto step = [&](int d, int s, int m) {
+        const float4 v = xr[d][s >> 2][m];
+        return (s & 3) == 0 ? v.x : (s & 3) == 1 ? v.y : (s & 3) == 2 ? v.z : v.w;
+    };
+    v4f acc[MP];
 #pragma unroll
-                for (int m = 0; m < NMF; m++) {
-                    const int pm = min(p0 + 4 * m, a.ldx - 4);
-                    st[i][m] = *reinterpret_cast<const float4*>(a.x + (size_t)k * ldx + pm);
-                }
-            }
+    for (int m = 0; m < MP; m++) acc[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int d = 0; d < DC; d++) request(d, d);
+    int c = 0;
+    for (; 8 * (c + DC) <= nst; c += DC) {
+#pragma unroll
+        for (int d = 0; d < DC; d++) {
+#pragma unroll
+            for (int s = 0; s < 8; s++)
+#pragma unroll
+                for (int m = 0; m < MP; m++)
+                    acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(wval<F32W>(wr[d], s), step(d, s, m), acc[m], 0, 0, 0);
+            request(c + d + DC, d);
         }
-        if (c >= 0) {
-            const float* xc = &xs[wv][c & 1][0][0];
-            const int kb0 = c * (KC / 8);
-#pragma unroll
-            for (int u = 0; u < KC / 8; u++) {   // the ring slot u % DW is static (KC / 8 is a multiple of DW)
-                const int kb = kb0 + u, kn = kb + DW < nk8 ? kb + DW : nk8 - 1;
-                float w[8];
-                wconv<F32W>(wq[u % DW], w);
-                wq[u % DW] = wload<F32W>(a.W.w, (size_t)kn * rp + rr);
-                if (kb < nk8) {
-                    float xv[NMF][8];
-#pragma unroll
-                    for (int m = 0; m < NMF; m++) {
-                        const float* xp = xc + (4 * m + q) * KCP + 8 * u;
-                        const float4 x0 = *reinterpret_cast<const float4*>(xp), x1 = *reinterpret_cast<const float4*>(xp + 4);
-                        xv[m][0] = x0.x; xv[m][1] = x0.y; xv[m][2] = x0.z; xv[m][3] = x0.w;
-                        xv[m][4] = x1.x; xv[m][5] = x1.y; xv[m][6] = x1.z; xv[m][7] = x1.w;
-                    }
-#pragma unroll
-                    for (int j = 0; j < 8; j++)
-#pragma unroll
-                        for (int m = 0; m < NMF; m++) acc[m] = __builtin_amdgcn_mfma_f32_4x4x1f32(w[j], xv[m][j], acc[m], 0, 0, 0);
-                }
-            }
-        }
-        __builtin_amdgcn_wave_barrier();
-        if (c + 1 < nch) {
-#pragma unroll
-            for (int i = 0; i < KC / 64; i++)
-#pragma unroll
-                for (int m = 0; m < NMF; m++) {
-                    float* xw = &xs[wv][(c + 1) & 1][4 * m][lane + 64 * i];
-                    xw[0] = st[i][m].x;
-                    xw[KCP] = st[i][m].y;
-                    xw[2 * KCP] = st[i][m].z;
-                    xw[3 * KCP] = st[i][m].w;
-                }
-        }
-        __builtin_amdgcn_wave_barrier();
     }
-    // lane l holds rows rb .. rb + 3 of position p0 + 4 m + l % 4 (rb = the workgroup's first row + 4 (l / 4))
-    const int rb = blockIdx.x * 64 + 4 * (lane >> 2);
+#pragma unroll
+    for (int d = 0; d < DC; d++)
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+            if (8 * (c + d) + s < nst) {
+#pragma unroll
+                for (int m = 0; m < MP; m++)
+                    acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(wval<F32W>(wr[d], s), step(d, s, m), acc[m], 0, 0, 0);
+            }
+    // lane l holds rows rb .. rb + 3 of position p0 + 16 m + l % 16
+    const int rb = 16 * tile + 4 * lq;
     if (EXPE && lane < 32) eE[wv][EXPE ? lane : 0] = et;
     __builtin_amdgcn_wave_barrier();
     const uint64_t* etab = eE[wv];
-    const bool xt = a.xt_out;
-    const int pend = xt ? min(a.ldx, a.ldo) : a.P;   // the feature-major output also fills the padded positions
+    const int kind = a.out_kind;
+    const int pend = kind != EO_POS ? min(a.ldx, a.ldo) : a.P;   // feature-major outputs also fill the padded positions
     auto put = [&](int row, int p, float v) {
-        float* d = xt ? a.out + (size_t)row * a.ldo + p : a.out + (size_t)p * a.ldo + row;
+        float* d = kind == EO_POS ? a.out + (size_t)p * a.ldo + row : kind == EO_FEAT ? a.out + (size_t)row * a.ldo + p
+                                                                                     : a.out + xat(row, p, a.ldo);
         *d = EPI == EE_ADD ? *d + v : v;
     };
 #pragma unroll
-    for (int m = 0; m < NMF; m++) {
-        const int p = p0 + 4 * m + q;
-        if constexpr (EPI == EE_GLU) {   // rows 0-7 of each 16 are gates, 8-15 the matching ups (lanes + 8)
+    for (int m = 0; m < MP; m++) {
+        const int p = p0 + 16 * m + li;
+        if constexpr (EPI == EE_GLU) {   // rows 0-7 of each 16 are gates, 8-15 the matching ups (lanes + 32)
             v4f up;
 #pragma unroll
-            for (int i = 0; i < 4; i++) up[i] = __shfl_xor(acc[m][i], 8);
-            if ((lane & 8) == 0 && p < pend) {
+            for (int i = 0; i < 4; i++) up[i] = __shfl_xor(acc[m][i], 32);
+            if (lq < 2 && p < pend) {
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const int row = rb + i, ro = (row >> 4) * 8 + (row & 7);
+                    const int ro = 8 * tile + 4 * lq + i;
                     if (ro < a.W.rows / 2) put(ro, p, silu_t(acc[m][i], etab) * up[i]);
                 }
             }
@@ -200,12 +189,21 @@ __global__ __launch_bounds__(ET) void k_etab(etab_args a) {
     }
 }
 
+// (these fill table inputs: a thread writes the four features e, e + 4, e + 8, e + 12 that are one 16-byte word)
+__device__ __forceinline__ int quad_feature(int g) { return 16 * (g >> 2) + (g & 3); }
+
 __global__ __launch_bounds__(ET) void k_eframes(const float* pcm, int n, const float* hann, int n_fft, int hop,
                                                 int n_fr, float* fx, int ldf) {
-    const int fr = blockIdx.x * ET + threadIdx.x, k = blockIdx.y;
+    const int fr = blockIdx.x * ET + threadIdx.x, k0 = quad_feature(blockIdx.y);
     if (fr >= ldf) return;
-    const long i = (long)fr * hop + k;
-    fx[(size_t)k * ldf + fr] = fr < n_fr && i < n ? hann[k] * pcm[i] : 0.0f;
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int k = k0 + 4 * q;
+        const long i = (long)fr * hop + k;
+        v[q] = k < n_fft && fr < n_fr && i < n ? hann[k] * pcm[i] : 0.0f;
+    }
+    *reinterpret_cast<float4*>(fx + xat(k0, fr, ldf)) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
 // imi sums all n_bin terms in bin order; a term with a zero filter weight is fma(0, pw, s) = s exactly (pw is a sum of
@@ -255,33 +253,43 @@ __global__ __launch_bounds__(ET) void k_econv0(const float* mel, int n_fr, int n
 
 __global__ __launch_bounds__(ET) void k_edw(const float* in, int Ti, int Fi, int ldi, const float* w9, const float* b,
                                             int C, int To, int Fo, float* out, int ldo) {
-    const int i = blockIdx.x * ET + threadIdx.x, c = blockIdx.y;
+    const int i = blockIdx.x * ET + threadIdx.x, c0 = quad_feature(blockIdx.y);
     if (i >= To * Fo) return;
     const int t = i / Fo, f = i - t * Fo;
-    const float* src = in + (size_t)c * ldi;
-    float v[9];
+    int at[9];
     bool ok[9];
 #pragma unroll
     for (int j = 0; j < 9; j++) {
         const int ti = 2 * t + j % 3 - 1, fi = 2 * f + j / 3 - 1;
         ok[j] = ti >= 0 && ti < Ti && fi >= 0 && fi < Fi;
         const int tc = ti < 0 ? 0 : ti >= Ti ? Ti - 1 : ti, fc = fi < 0 ? 0 : fi >= Fi ? Fi - 1 : fi;
-        v[j] = src[(size_t)tc * Fi + fc];
+        at[j] = tc * Fi + fc;
     }
-    float o = b[c];
+    float o[4];
 #pragma unroll
-    for (int j = 0; j < 9; j++) {
-        const float u = fmaf(v[j], w9[(size_t)j * C + c], o);
-        o = ok[j] ? u : o;
+    for (int q = 0; q < 4; q++) {
+        const int c = min(c0 + 4 * q, C - 1);
+        const float* src = in + (size_t)c * ldi;
+        o[q] = b[c];
+#pragma unroll
+        for (int j = 0; j < 9; j++) {
+            const float u = fmaf(src[at[j]], w9[(size_t)j * C + c], o[q]);
+            o[q] = ok[j] ? u : o[q];
+        }
     }
-    out[(size_t)c * ldo + (size_t)t * Fo + f] = o;
+    *reinterpret_cast<float4*>(out + xat(c0, i, ldo)) = make_float4(o[0], o[1], o[2], o[3]);
 }
 
-__global__ __launch_bounds__(ET) void k_eflat(const float* a, int lda, int F8, int P, float* xf, int ldf) {
-    const int p = blockIdx.x * ET + threadIdx.x, k = blockIdx.y;
+__global__ __launch_bounds__(ET) void k_eflat(const float* a, int lda, int K, int F8, int P, float* xf, int ldf) {
+    const int p = blockIdx.x * ET + threadIdx.x, k0 = quad_feature(blockIdx.y);
     if (p >= ldf) return;
-    const int c = k / F8, f = k - c * F8;
-    xf[(size_t)k * ldf + p] = p < P ? a[(size_t)c * lda + (size_t)p * F8 + f] : 0.0f;
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int k = min(k0 + 4 * q, K - 1), c = k / F8, f = k - c * F8;
+        v[q] = p < P ? a[(size_t)c * lda + (size_t)p * F8 + f] : 0.0f;
+    }
+    *reinterpret_cast<float4*>(xf + xat(k0, p, ldf)) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
 // a workgroup is 16 positions x 64 features: each wave forms 4 positions' scales in imi's order (every workgroup of a
@@ -297,15 +305,19 @@ __global__ __launch_bounds__(ET) void k_enorm(const float* x, const float* w, in
     __syncthreads();
     const int pl = threadIdx.x & 15, p = p0 + pl;
     const float s = sc[pl];
-    for (int e = e0 + (threadIdx.x >> 4); e < e0 + 64 && e < E; e += ET / 16)
-        h[(size_t)e * ldh + p] = p < P ? x[(size_t)p * E + e] * s * w[e] : 0.0f;
+    const int e = e0 + quad_feature((int)threadIdx.x >> 4);
+    if (e >= E) return;   // (E is a multiple of 32)
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) v[q] = p < P ? x[(size_t)p * E + e + 4 * q] * s * w[e + 4 * q] : 0.0f;
+    *reinterpret_cast<float4*>(h + xat(e, p, ldh)) = make_float4(v[0], v[1], v[2], v[3]);
 }
 
 __global__ __launch_bounds__(ET) void k_econv(const float* big, int ld, const float* w, int E, int d_conv, int P,
                                               float* act, int lda) {
     const int e = blockIdx.x * ET + threadIdx.x, p = blockIdx.y;
     if (e >= E) return;
-    if (p >= P) { act[(size_t)e * lda + p] = 0.0f; return; }
+    if (p >= P) { act[xat(e, p, lda)] = 0.0f; return; }
     float co = 0.0f;
     for (int k = 0; k < d_conv; k++) {
         const int t = p - (d_conv - 1) + k;
@@ -313,7 +325,7 @@ __global__ __launch_bounds__(ET) void k_econv(const float* big, int ld, const fl
         const float* rw = big + (size_t)t * ld;
         co = fmaf(w[(size_t)k * E + e], rw[e] * rw[2 * E + e], co);
     }
-    act[(size_t)e * lda + p] = big[(size_t)p * ld + E + e] * co;
+    act[xat(e, p, lda)] = big[(size_t)p * ld + E + e] * co;
 }
 
 // one wave per (position, head slot): the n_head query heads, then the n_kv key heads
@@ -373,7 +385,7 @@ __global__ __launch_bounds__(ET) void k_eattn(const float* big, int ld, int n_he
     for (int i = lane; i < D; i += 64) {
         float o = 0.0f;
         for (int t = 0; t < nk; t++) o = fmaf(es[wv][t], big[(size_t)(s0 + t) * ld + Hq + Hk + kv * D + i], o);
-        act[(size_t)(hh * D + i) * lda + p] = o / sum;
+        act[xat(hh * D + i, p, lda)] = o / sum;
     }
 }
 
@@ -386,7 +398,7 @@ __global__ __launch_bounds__(ET) void k_efinal(const float* x, const float* post
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, p = blockIdx.x * (ET / 64) + wv;
     if (p >= ldh) return;
     if (p >= P) {
-        for (int e = lane; e < E; e += 64) h[(size_t)e * ldh + p] = 0.0f;
+        for (int e = lane; e < E; e += 64) h[xat(e, p, ldh)] = 0.0f;
         return;
     }
     float* hs = hs_all + (size_t)wv * E;
@@ -408,28 +420,28 @@ __global__ __launch_bounds__(ET) void k_efinal(const float* x, const float* post
     __builtin_amdgcn_wave_barrier();
     const double mu = st[wv][0];
     const float inv = (float)st[wv][1];
-    for (int e = lane; e < E; e += 64) h[(size_t)e * ldh + p] = fmaf((float)((double)hs[e] - mu) * inv, ln_w[e], ln_b[e]);
+    for (int e = lane; e < E; e += 64) h[xat(e, p, ldh)] = fmaf((float)((double)hs[e] - mu) * inv, ln_w[e], ln_b[e]);
 }
 
 inline unsigned blocks(long n) { return (unsigned)((n + ET - 1) / ET); }
+inline unsigned quads(int n) { return (unsigned)((n + 15) / 16 * 4); }   // feature quads (quad_feature)
 
 }  // namespace
 
 hipError_t launch_etab(int epi, const etab_args& a, hipStream_t s) {
-    if (a.W.cols % 8 || a.W.rows_pad % 8 || a.ldx % 16 || (a.xt_out && a.ldo % 4) ||
-        (epi == EE_GLU && a.W.rows_pad % 16))
-        return hipErrorInvalidValue;
+    if (a.W.cols % 8 || a.W.cols < 8 || a.W.rows_pad % 16 || a.ldx % 16 || a.ldx < 16 ||
+        (a.out_kind == EO_FEAT && a.ldo % 4) || (a.out_kind == EO_TABLE && a.ldo % 16)) return hipErrorInvalidValue;
     const unsigned gx = (unsigned)((a.W.rows_pad + 63) / 64);
-    // position quads per wave: the most that keeps enough waves in flight (the chains are as long as the table is wide)
-    const auto waves = [&](int nmf) { return 4L * gx * ((a.ldx + 16 * nmf - 1) / (16 * nmf)); };
-    const int nmf = waves(4) >= 2048 ? 4 : waves(2) >= 2048 ? 2 : 1;
-    const dim3 grid(gx, (unsigned)((a.ldx + 16 * nmf - 1) / (16 * nmf)));
+    // position tiles per wave: the most that keeps enough waves in flight
+    const auto waves = [&](int mp) { return 4L * gx * ((a.ldx + 16 * mp - 1) / (16 * mp)); };
+    const int mp = waves(4) >= 2048 ? 4 : waves(2) >= 2048 ? 2 : 1;
+    const dim3 grid(gx, (unsigned)((a.ldx + 16 * mp - 1) / (16 * mp)));
 #define SH_ETAB(E)                                                                                        \
     case E:                                                                                               \
         if (a.W.f32) {                                                                                    \
-            if (nmf == 4) SH_ETAB_MF(E, true, 4); else if (nmf == 2) SH_ETAB_MF(E, true, 2); else SH_ETAB_MF(E, true, 1); \
+            if (mp == 4) SH_ETAB_MF(E, true, 4); else if (mp == 2) SH_ETAB_MF(E, true, 2); else SH_ETAB_MF(E, true, 1); \
         } else {                                                                                          \
-            if (nmf == 4) SH_ETAB_MF(E, false, 4); else if (nmf == 2) SH_ETAB_MF(E, false, 2); else SH_ETAB_MF(E, false, 1); \
+            if (mp == 4) SH_ETAB_MF(E, false, 4); else if (mp == 2) SH_ETAB_MF(E, false, 2); else SH_ETAB_MF(E, false, 1); \
         }                                                                                                 \
         break;
 #define SH_ETAB_MF(E, F, N) hipLaunchKernelGGL((k_etab<E, F, N>), grid, dim3(ET), 0, s, a)
@@ -444,7 +456,7 @@ hipError_t launch_etab(int epi, const etab_args& a, hipStream_t s) {
 
 hipError_t launch_eframes(const float* pcm, int n, const float* hann, int n_fft, int hop, int n_fr, float* fx, int ldf,
                           hipStream_t s) {
-    hipLaunchKernelGGL(k_eframes, dim3(blocks(ldf), n_fft), dim3(ET), 0, s, pcm, n, hann, n_fft, hop, n_fr, fx, ldf);
+    hipLaunchKernelGGL(k_eframes, dim3(blocks(ldf), quads(n_fft)), dim3(ET), 0, s, pcm, n, hann, n_fft, hop, n_fr, fx, ldf);
     return hipGetLastError();
 }
 hipError_t launch_emel(const float* pw, int ldp, const float* fb, const int2* span, int n_bin, int n_mel, int n_fr,
@@ -462,11 +474,11 @@ hipError_t launch_econv0(const float* mel, int n_fr, int n_mel, const float* w9,
 hipError_t launch_edw(const float* in, int Ti, int Fi, int ldi, const float* w9, const float* b, int C, float* out,
                       int ldo, hipStream_t s) {
     const int To = (Ti + 1) / 2, Fo = Fi / 2;
-    hipLaunchKernelGGL(k_edw, dim3(blocks((long)To * Fo), C), dim3(ET), 0, s, in, Ti, Fi, ldi, w9, b, C, To, Fo, out, ldo);
+    hipLaunchKernelGGL(k_edw, dim3(blocks((long)To * Fo), quads(C)), dim3(ET), 0, s, in, Ti, Fi, ldi, w9, b, C, To, Fo, out, ldo);
     return hipGetLastError();
 }
 hipError_t launch_eflat(const float* a, int lda, int C, int F8, int P, float* xf, int ldf, hipStream_t s) {
-    hipLaunchKernelGGL(k_eflat, dim3(blocks(ldf), C * F8), dim3(ET), 0, s, a, lda, F8, P, xf, ldf);
+    hipLaunchKernelGGL(k_eflat, dim3(blocks(ldf), quads(C * F8)), dim3(ET), 0, s, a, lda, C * F8, F8, P, xf, ldf);
     return hipGetLastError();
 }
 hipError_t launch_enorm(const float* x, const float* w, int E, int P, float eps, float* h, int ldh, hipStream_t s) {

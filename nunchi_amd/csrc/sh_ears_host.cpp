@@ -34,6 +34,7 @@ struct elayer {
 constexpr int N_FFT = 400, HOP = 160, N_BIN = N_FFT / 2 + 1;
 
 inline int pad16(long v) { return (int)((v + 15) / 16 * 16); }
+inline int pad32(long v) { return (int)((v + 31) / 32 * 32); }
 
 struct geom {   // imi/core/ears.cpp:201-205
     int n_fr, T2, F2, T4, F4, P, F8;
@@ -88,28 +89,30 @@ void release(sh_ears* e) {
     delete e;
 }
 
-// one float table in the device layout: [cols / 8][rows_pad][8] of the file's element type
+// one float table in the device layout (sh_ears.h), of the file's element type
 struct tplan {
     std::vector<std::pair<const gg_tensor*, int>> rows;   // (tensor, row)
     const float* dense = nullptr;                          // or a dense fp32 [rows][cols] host matrix
     int n_dense = 0, cols = 0;
     bool f32 = false;
     etab* dst = nullptr;
+    size_t count() const { return dense ? n_dense : rows.size(); }
     size_t bytes() const {
-        const size_t nr = dense ? n_dense : rows.size();
-        return (nr + 7) / 8 * 8 * cols * (f32 ? 4 : 2);
+        const size_t nr = count();
+        return (nr + 15) / 16 * 16 * ((cols + 31) / 32 * 32) * (f32 ? 4 : 2);
     }
 };
 
 void fill_table(const tplan& t, uint8_t* o) {
-    const int nr = t.dense ? t.n_dense : (int)t.rows.size(), rp = (nr + 7) / 8 * 8, K = t.cols;
+    const int nr = t.dense ? t.n_dense : (int)t.rows.size(), rp = (nr + 15) / 16 * 16, K = t.cols;
     memset(o, 0, t.bytes());
     for (int r = 0; r < nr; r++) {
         const uint8_t* src = t.dense ? nullptr
                                      : static_cast<const uint8_t*>(t.rows[r].first->data) +
                                            (size_t)t.rows[r].second * t.rows[r].first->nb[1];
         for (int k = 0; k < K; k++) {
-            const size_t at = ((size_t)(k / 8) * rp + r) * 8 + k % 8;
+            const size_t tile = (size_t)(k / 32) * (rp / 16) + r / 16, lane = (k % 4) * 16 + r % 16, v = k % 32 / 4;
+            const size_t at = t.f32 ? ((tile * 2 + v / 4) * 64 + lane) * 4 + v % 4 : (tile * 64 + lane) * 8 + v;
             if (t.f32) {
                 const float v = t.dense ? t.dense[(size_t)r * K + k] : reinterpret_cast<const float*>(src)[k];
                 memcpy(o + at * 4, &v, 4);
@@ -128,9 +131,9 @@ bool is_table(const gg_tensor* t, int64_t cols, int64_t rows) {
 }
 
 int run_table(sh_ears* e, int epi, const etab& W, const float* x, int ldx, int P, const float* bias, float* out, int ldo,
-              bool xt) {
+              int kind) {
     etab_args a{};
-    a.W = W; a.x = x; a.ldx = ldx; a.P = P; a.bias = bias; a.out = out; a.ldo = ldo; a.xt_out = xt;
+    a.W = W; a.x = x; a.ldx = ldx; a.P = P; a.bias = bias; a.out = out; a.ldo = ldo; a.out_kind = kind;
     ECHK(launch_etab(epi, a, e->stream));
     return SH_OK;
 }
@@ -148,20 +151,20 @@ int ensure_work(sh_ears* e, int n) {
               P8 = pad16((long)g.P * g.F8);
     std::vector<size_t> sz = {
         (size_t)n,                                        // pcm
-        (size_t)N_FFT * Pf,                               // fx
+        (size_t)pad32(N_FFT) * Pf,                               // fx
         (size_t)N_BIN * Pf,                               // pw
         (size_t)g.n_fr * I.n_mel,                         // mel
         (size_t)C * g.T2 * g.F2,                          // a0
-        (size_t)C * P4,                                   // a1
+        (size_t)pad32(C) * P4,                            // a1
         (size_t)C * P4,                                   // a2
-        (size_t)C * P8,                                   // a3
+        (size_t)pad32(C) * P8,                            // a3
         (size_t)C * P8,                                   // a4
-        (size_t)C * g.F8 * Pp,                            // xf
+        (size_t)pad32(C * g.F8) * Pp,                     // xf
         (size_t)g.P * E,                                  // x
         (size_t)std::max(E, I.n_embd) * Pp,               // h
         (size_t)g.P * e->big_w,                           // big
-        (size_t)std::max({I.n_ff, I.n_head * std::max(I.head_dim, 1), E}) * Pp,   // act
-        (size_t)e->n_mid * Pp,                            // proj
+        (size_t)pad32(std::max({I.n_ff, I.n_head * std::max(I.head_dim, 1), E})) * Pp,   // act
+        (size_t)pad32(e->n_mid) * Pp,                       // proj
         (size_t)g.P * I.n_out,                            // out
         (size_t)g.P * std::max(I.head_dim, 2),            // cs (float2 [P][D / 2])
     };
@@ -198,36 +201,36 @@ int enqueue_encode(sh_ears* e, int n) {
     hipStream_t s = e->stream;
     // mel (ears.cpp:211-238)
     ECHK(launch_eframes(e->pcm, n, e->hann, N_FFT, HOP, g.n_fr, e->fx, Pf, s));
-    RUN(run_table(e, EE_POWER, e->dft, e->fx, Pf, g.n_fr, nullptr, e->pw, Pf, true));
+    RUN(run_table(e, EE_POWER, e->dft, e->fx, Pf, g.n_fr, nullptr, e->pw, Pf, EO_FEAT));
     ECHK(launch_emel(e->pw, Pf, e->fb, e->fb_span, N_BIN, I.n_mel, g.n_fr, e->mel, s));
     // downsampler (ears.cpp:241-296), channel-major
     ECHK(launch_econv0(e->mel, g.n_fr, I.n_mel, e->c0_w, e->c0_b, C, e->a0, s));
     ECHK(launch_edw(e->a0, g.T2, g.F2, g.T2 * g.F2, e->c2_w, e->c2_b, C, e->a1, P4, s));
-    RUN(run_table(e, EE_SILU, e->c3, e->a1, P4, g.T4 * g.F4, e->c3_b, e->a2, P4, true));
+    RUN(run_table(e, EE_SILU, e->c3, e->a1, P4, g.T4 * g.F4, e->c3_b, e->a2, P4, EO_FEAT));
     ECHK(launch_edw(e->a2, g.T4, g.F4, P4, e->c5_w, e->c5_b, C, e->a3, P8, s));
-    RUN(run_table(e, EE_SILU, e->c6, e->a3, P8, g.P * g.F8, e->c6_b, e->a4, P8, true));
+    RUN(run_table(e, EE_SILU, e->c6, e->a3, P8, g.P * g.F8, e->c6_b, e->a4, P8, EO_FEAT));
     ECHK(launch_eflat(e->a4, P8, C, g.F8, g.P, e->xf, Pp, s));
-    RUN(run_table(e, EE_STORE, e->pre, e->xf, Pp, g.P, e->pre_b, e->x, E, false));
+    RUN(run_table(e, EE_STORE, e->pre, e->xf, Pp, g.P, e->pre_b, e->x, E, EO_POS));
     // layers (ears.cpp:302-370)
     for (const elayer& L : e->layers) {
         ECHK(launch_enorm(e->x, L.ln1, E, g.P, e->eps, e->h, Pp, s));
         const int ld = L.in.rows;
-        RUN(run_table(e, EE_STORE, L.in, e->h, Pp, g.P, nullptr, e->big, ld, false));
+        RUN(run_table(e, EE_STORE, L.in, e->h, Pp, g.P, nullptr, e->big, ld, EO_POS));
         if (!L.attn) {
             ECHK(launch_econv(e->big, ld, L.conv_w, E, I.d_conv, g.P, e->act, Pp, s));
         } else {
             ECHK(launch_eqk(e->big, ld, I.n_head, I.n_head_kv, D, L.q_norm, L.k_norm, e->cs, g.P, e->eps, s));
             ECHK(launch_eattn(e->big, ld, I.n_head, I.n_head_kv, D, I.window, g.P, e->act, Pp, s));
         }
-        RUN(run_table(e, EE_ADD, L.out, e->act, Pp, g.P, nullptr, e->x, E, false));
+        RUN(run_table(e, EE_ADD, L.out, e->act, Pp, g.P, nullptr, e->x, E, EO_POS));
         ECHK(launch_enorm(e->x, L.ln2, E, g.P, e->eps, e->h, Pp, s));
-        RUN(run_table(e, EE_GLU, L.gate_up, e->h, Pp, g.P, nullptr, e->act, Pp, true));
-        RUN(run_table(e, EE_ADD, L.down, e->act, Pp, g.P, nullptr, e->x, E, false));
+        RUN(run_table(e, EE_GLU, L.gate_up, e->h, Pp, g.P, nullptr, e->act, Pp, EO_TABLE));
+        RUN(run_table(e, EE_ADD, L.down, e->act, Pp, g.P, nullptr, e->x, E, EO_POS));
     }
     // last norm, LayerNorm, projector (ears.cpp:372-403)
     ECHK(launch_efinal(e->x, e->post_ln, e->ln_w, e->ln_b, E, g.P, e->eps, e->h, Pp, s));
-    RUN(run_table(e, EE_GELU, e->mlp1, e->h, Pp, g.P, e->mlp1_b, e->proj, Pp, true));
-    RUN(run_table(e, EE_STORE, e->mlp3, e->proj, Pp, g.P, e->mlp3_b, e->out, I.n_out, false));
+    RUN(run_table(e, EE_GELU, e->mlp1, e->h, Pp, g.P, e->mlp1_b, e->proj, Pp, EO_TABLE));
+    RUN(run_table(e, EE_STORE, e->mlp3, e->proj, Pp, g.P, e->mlp3_b, e->out, I.n_out, EO_POS));
     return SH_OK;
 }
 
@@ -449,7 +452,7 @@ int sh_ears_load(int device, const char* path, sh_ears** out) {   // imi/core/ea
     whole(m3, &e->mlp3);
 
     size_t need = 0, tbytes = 0;
-    for (const tplan& t : tabs) { need += (t.bytes() + 255) / 256 * 256; tbytes += t.bytes(); }
+    for (const tplan& t : tabs) { need += (t.bytes() + 255) / 256 * 256; tbytes += (t.count() + 7) / 8 * 8 * t.cols * (t.f32 ? 4 : 2); }
     for (const vec& v : vecs) need += ((size_t)v.n * 4 + 255) / 256 * 256;
     I.table_bytes = (long long)tbytes;
     e->info = I;
@@ -462,7 +465,7 @@ int sh_ears_load(int device, const char* path, sh_ears** out) {   // imi/core/ea
         const int nr = t.dense ? t.n_dense : (int)t.rows.size();
         t.dst->w = e->mem + off;
         t.dst->rows = nr;
-        t.dst->rows_pad = (nr + 7) / 8 * 8;
+        t.dst->rows_pad = (nr + 15) / 16 * 16;
         t.dst->cols = t.cols;
         t.dst->f32 = t.f32;
         off += (t.bytes() + 255) / 256 * 256;

@@ -33,6 +33,20 @@ def test_tiny_ears_matches_oracle(tiny_ears, n):
     assert oracle.rel(out, ref) < TOL, oracle.rel(out, ref)
 
 
+@pytest.mark.parametrize("n", [300, 5 * 16000 + 7])
+def test_odd_table_sizes_match_oracle(model_dir, n):
+    """Tables whose rows and columns end inside a 16-row tile and a 32-column chunk (8, 24, 40 and 264 columns, 264 rows)."""
+    import nunchi_amd
+    from nunchi_amd import synth
+    shape = synth.EarsShape(n_mel=24, n_ch=8, n_embd=96, n_ff=40, n_head=3, n_head_kv=1, head_dim=32, layers="ca",
+                            window=5, n_out=264)
+    path = synth.cached("ears", shape, 4, model_dir)
+    out = nunchi_amd.Ears(path).encode(synth.clip(n, 8))
+    ref = oracle.Ears(path, threads=4).encode(synth.clip(n, 8))
+    assert out.shape == ref.shape
+    assert oracle.rel(out, ref) < TOL, oracle.rel(out, ref)
+
+
 def test_encode_repeats_and_shrinks(tiny_ears):
     """A longer clip, a shorter one (the work buffers are kept), then the first again: bit for bit the same rows."""
     import nunchi_amd
