@@ -159,128 +159,16 @@ __global__ __launch_bounds__(256) void k_pf_cut(pf_cutk_args a) {
 }
 
 // ---------------------------------------------------------------- table products on the matrix cores
-// Workgroup tile 64 rows x 64 positions, wave tile 32 x 32 (2 x 2 products of 16 x 16 per 32-column block).
 // v_mfma_i32_16x16x32_i8 operands: lane l holds row / position l % 16, columns 8 (l / 16) .. + 7 of the block;
 // the result's lane l holds rows 4 (l / 16) + i (i < 4) at position l % 16. The weight codes enter as they are
 // stored (0..15), the input as its int8 cut, so each product is imi's integer block sum exactly; then per (row,
 // position), block by block in order: acc = fma(float(isum), d * dx, acc), cor = fma(d, s, cor), and at the end
 // out = fma(-8, cor, acc) (imi/core/tables.cpp:419-454, the batch kernel imi's prefill uses); Q4_1 tables take the
 // block minimum m in the cor chain and end as acc + cor.
-template <int EPI, bool HM>
-__global__ __launch_bounds__(256) void k_pf_gemm(pf_gemm_args a) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int li = lane & 15, lq = lane >> 4;
-    const int rows = a.W.rows, n = a.n, nb = a.W.nb;
-    const int rbase = blockIdx.x * 64 + (w & 1) * 32, pbase = blockIdx.y * 64 + (w >> 1) * 32;
-    if (rbase >= rows || pbase >= n) return;   // whole waves; no barriers below
-    const uint8_t* codes = static_cast<const uint8_t*>(a.W.codes);
-    const uint16_t* scales = static_cast<const uint16_t*>(a.W.scales);
-    const uint16_t* mins = static_cast<const uint16_t*>(a.W.mins);
-    const uint8_t* ap[2];
-    const uint16_t* dp[2];
-    const uint16_t* mp[2];
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++) {
-        const int r = min(rbase + 16 * mt + li, rows - 1);              // operand row (clamped: results dropped)
-        ap[mt] = codes + (size_t)r * nb * 16 + (lq & 1) * 8;            // bytes 0-7 or 8-15 of the row's block
-        const int rd = min(rbase + 16 * mt + 4 * lq, rows - 4);         // first of the 4 result rows
-        dp[mt] = scales + (size_t)(rd >> 3) * nb * 8 + (rd & 7);
-        mp[mt] = HM ? mins + (size_t)(rd >> 3) * nb * 8 + (rd & 7) : dp[mt];
-    }
-    const int shift = (lq >> 1) * 4;   // columns 0-15: low nibbles, 16-31: high nibbles
-    int pp[2];
-#pragma unroll
-    for (int nt = 0; nt < 2; nt++) pp[nt] = min(pbase + 16 * nt + li, n - 1);
-
-    float acc[2][2][4], cor[2][2][4];
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) { acc[mt][nt][i] = 0.0f; cor[mt][nt][i] = 0.0f; }
-
-    // operands of block j, fetched one block ahead
-    uint2 ra[2], rs[2], rm[2];
-    long rb[2];
-    float fx[2], fs[2];
-    auto fetch = [&](int j) {
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++) {
-            ra[mt] = *reinterpret_cast<const uint2*>(ap[mt] + (size_t)j * 16);
-            rs[mt] = *reinterpret_cast<const uint2*>(dp[mt] + (size_t)j * 8);
-            if (HM) rm[mt] = *reinterpret_cast<const uint2*>(mp[mt] + (size_t)j * 8);
-        }
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++) {
-            const size_t o = (size_t)j * n + pp[nt];
-            rb[nt] = *reinterpret_cast<const long*>(a.in.q + o * 32 + lq * 8);
-            fx[nt] = a.in.d[o];
-            fs[nt] = a.in.s[o];
-        }
-    };
-    fetch(0);
-    for (int j = 0; j < nb; j++) {
-        const uint2 ca[2] = {ra[0], ra[1]}, cs[2] = {rs[0], rs[1]}, cm[2] = {HM ? rm[0] : rs[0], HM ? rm[1] : rs[1]};
-        const long cb[2] = {rb[0], rb[1]};
-        const float cx[2] = {fx[0], fx[1]}, cz[2] = {fs[0], fs[1]};
-        if (j + 1 < nb) fetch(j + 1);
-        i32x4 isum[2][2];
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++) {
-            const unsigned lo = (ca[mt].x >> shift) & 0x0F0F0F0Fu, hi = (ca[mt].y >> shift) & 0x0F0F0F0Fu;
-            const long av = (long)((unsigned long)lo | ((unsigned long)hi << 32));
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++)
-                isum[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, cb[nt], i32x4{0, 0, 0, 0}, 0, 0, 0);
-        }
-#pragma unroll
-        for (int mt = 0; mt < 2; mt++) {
-            const float dd[4] = {h2f((uint16_t)(cs[mt].x & 0xFFFFu)), h2f((uint16_t)(cs[mt].x >> 16)),
-                                 h2f((uint16_t)(cs[mt].y & 0xFFFFu)), h2f((uint16_t)(cs[mt].y >> 16))};
-            const float mm[4] = {h2f((uint16_t)(cm[mt].x & 0xFFFFu)), h2f((uint16_t)(cm[mt].x >> 16)),
-                                 h2f((uint16_t)(cm[mt].y & 0xFFFFu)), h2f((uint16_t)(cm[mt].y >> 16))};
-#pragma unroll
-            for (int nt = 0; nt < 2; nt++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    acc[mt][nt][i] = fmaf((float)isum[mt][nt][i], dd[i] * cx[nt], acc[mt][nt][i]);
-                    cor[mt][nt][i] = fmaf(mm[i], cz[nt], cor[mt][nt][i]);
-                }
-        }
-    }
-#pragma unroll
-    for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-        for (int nt = 0; nt < 2; nt++) {
-            const int p = pbase + 16 * nt + li, r0 = rbase + 16 * mt + 4 * lq;
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = HM ? acc[mt][nt][i] + cor[mt][nt][i] : fmaf(-8.0f, cor[mt][nt][i], acc[mt][nt][i]);
-            if (EPI == EPI_SWIGLU) {
-                // rows 0-7 of the 16-row tile are a gate group, rows 8-15 the matching up group (lanes + 32)
-                float up[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) up[i] = __shfl_xor(v[i], 32);
-                if (lq < 2 && p < n) {
-                    float* o = a.out + (size_t)p * a.out_ld + (rbase + 16 * mt) / 2 + 4 * lq;
-#pragma unroll
-                    for (int i = 0; i < 4; i++) o[i] = silu(v[i]) * up[i];
-                }
-            } else if (p < n) {
-                float* o = a.out + (size_t)p * a.out_ld + r0;
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (r0 + i < rows) o[i] = v[i];
-            }
-        }
-}
-
-// LDS-staged form of the same product (taken when nb is a multiple of KC): per workgroup the operands of KC blocks
+// Per workgroup the operands of KC blocks
 // (64 rows of codes, their scales and, for Q4_1, minima; 64 positions of input codes and their (d, s)) are fetched
 // with wide coalesced loads into registers while the waves run the previous KC blocks from LDS, then stored to the
-// other half of a double buffer, the codes already split into their low and high nibbles. The per-(row, position)
-// operations and their order are k_pf_gemm's; two of the three fp32 operations per (row, position, block) run on
+// other half of a double buffer, the codes already split into their low and high nibbles. Two of the three fp32 operations per (row, position, block) run on
 // the matrix cores as K = 1 outer products, v_mfma_f32_16x16x1_4b_f32, whose four 16 x 16 blocks are the wave's
 // (row tile, position tile) pairs: dd = d x dx (accumulator 0) and cor = fma(d, s, cor) (the running cor as the
 // accumulator, one product per block in block order). That operation rounds once, like fmaf: it equals the VALU's
@@ -289,7 +177,12 @@ __global__ __launch_bounds__(256) void k_pf_gemm(pf_gemm_args a) {
 // fma(float(isum), dd, acc) stays on the VALU. A workgroup is 4 waves over 64 rows x 2 PW positions, a wave 32 rows x
 // PW positions: PW = 32 for tables with enough rows, 16 for the narrow ones (2048 rows: two waves per SIMD instead of
 // one), whose matrix-core blocks for the missing position tile are computed on a repeated position and dropped.
-template <int EPI, bool HM, int KC, int PW>
+// TAIL: block counts that are no multiple of KC. The last chunk's missing blocks re-read the last block and are staged
+// with zero codes and scales, which add +0 to chains that are never -0; the clamps cost the whole chunks' path about 3 %
+// (16384 x 2048 at 448 positions 74.9 -> 77.1 us), so that one is compiled without them. Against an unstaged product of
+// the same wave tiles: 4096 x 2080 at 448 / 100 / 17 positions 42.9 / 23.8 / 22.0 -> 37.6 / 15.5 / 14.4 us, 1024 x 8160
+// at 64 79.5 -> 48.1, 16384 x 288 at 512 39.1 -> 33.4.
+template <int EPI, bool HM, int KC, int PW, bool TAIL>
 __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_lds(pf_gemm_args a) {
     typedef float v16f __attribute__((ext_vector_type(16)));
     constexpr int P = 2 * PW, NTW = PW / 16;          // positions per workgroup; 16-position tiles per wave
@@ -301,7 +194,7 @@ __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_
     __shared__ float2 sX[2][KC][P];         // (d, s) of position p's block j
     __shared__ uint64_t sE[EPI == EPI_SWIGLU ? 32 : 1];   // expf's table for the SwiGLU epilogue (an LDS copy)
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, li = lane & 15, lq = lane >> 4;
-    const int rows = a.W.rows, n = a.n, nb = a.W.nb, nch = nb / KC, ng = rows / 8;
+    const int rows = a.W.rows, n = a.n, nb = a.W.nb, nch = TAIL ? (nb + KC - 1) / KC : nb / KC, ng = rows / 8;
     const int r0 = blockIdx.x * 64, p0 = blockIdx.y * P, rl = (w & 1) * 32, pl = (w >> 1) * PW;
     // staging words per thread (the (d, s) pairs of a narrow tile need only the first P * KC threads)
     constexpr int NA = 64 * KC / 256, NBQ = P * KC * 2 / 256, NX = (P * KC + 255) / 256;
@@ -331,21 +224,29 @@ __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_
     float gxd[NX], gxs[NX];
     auto fetch = [&](int c) {
         const int j0 = c * KC;
+        // block j0 + o of the table (its source already o blocks on), or with TAIL its last one
+        auto at = [&](int o) -> ptrdiff_t { return TAIL ? min(j0, nb - 1 - o) : j0; };
 #pragma unroll
-        for (int q = 0; q < NA; q++) ga[q] = pa[q][j0];
+        for (int q = 0; q < NA; q++) ga[q] = pa[q][at((t + 256 * q) % KC)];
 #pragma unroll
-        for (int q = 0; q < NBQ; q++) gb[q] = pb[q][(size_t)j0 * n * 2];
+        for (int q = 0; q < NBQ; q++) gb[q] = pb[q][at((t + 256 * q) / (2 * P)) * n * 2];
         if (t < 8 * KC) {
-            gd = ((const u32x4*)a.W.scales)[pdo + j0];
-            if (HM) gm = ((const u32x4*)a.W.mins)[pdo + j0];
+            gd = ((const u32x4*)a.W.scales)[pdo + at(t % KC)];
+            if (HM) gm = ((const u32x4*)a.W.mins)[pdo + at(t % KC)];
         }
 #pragma unroll
         for (int q = 0; q < NX; q++) {
-            gxd[q] = px[q][(size_t)j0 * n];
-            gxs[q] = px[q][(size_t)j0 * n + sdo];
+            const ptrdiff_t xo = at(min(t + 256 * q, P * KC - 1) / P) * n;
+            gxd[q] = px[q][xo];
+            gxs[q] = px[q][xo + (ptrdiff_t)sdo];
         }   // (threads past P * KC re-read the last pair; they store nothing)
     };
-    auto stash = [&](int buf) {
+    auto stash = [&](int buf, int c) {
+        if (TAIL && c * KC + t % KC >= nb) {
+#pragma unroll
+            for (int q = 0; q < NA; q++) ga[q] = u32x4{0, 0, 0, 0};
+            gd = gm = u32x4{0, 0, 0, 0};
+        }
 #pragma unroll
         for (int q = 0; q < NA; q++) {   // byte k of the record: low nibble of code byte k (k < 16), high of k - 16
             const int idx = t + 256 * q;
@@ -385,7 +286,7 @@ __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_
     const int orow = rl + 16 * (lane >> 5) + li, opos = pl + 16 * (NTW == 2 ? (lane >> 4) & 1 : 0) + li;
     const uint64_t et = EPI == EPI_SWIGLU ? kExp2Tab[t & 31] : 0;   // (requested first: its wait needs nothing later)
     fetch(0);
-    stash(0);
+    stash(0, 0);
     if (EPI == EPI_SWIGLU && t < 32) sE[t] = et;
     __syncthreads();
     for (int c = 0; c < nch; c++) {
@@ -422,7 +323,7 @@ __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_
                         acc[k] = fmaf((float)isum[mt][nt][i], dd[k], acc[k]);
                     }
         }
-        if (c + 1 < nch) stash(buf ^ 1);
+        if (c + 1 < nch) stash(buf ^ 1, c + 1);
         __syncthreads();
     }
     const int rbase = r0 + rl, pbase = p0 + pl;
@@ -1023,46 +924,33 @@ hipError_t launch_pf_rows(int mode, const pf_rows_args& a, hipStream_t s) {
 #ifndef PF_KC
 #define PF_KC 4   // blocks staged per step of the LDS-staged product
 #endif
-// SEOUL_HIP_PF_PLAIN=1 keeps the products on the unstaged kernel (a comparison switch)
-static bool getenv_pf_plain() {
-    static const int v = [] { const char* e = getenv("SEOUL_HIP_PF_PLAIN"); return e && e[0] == '1' ? 1 : 0; }();
-    return v != 0;
-}
 
 bool pf_swiglu_cut_takes(const pf_gemm_args& a) {
-    return a.n >= 1 && a.W.rows % 64 == 0 && a.out_ld * 2 == a.W.rows && a.W.nb % PF_KC == 0 && !getenv_pf_plain();
+    return a.n >= 1 && a.W.rows % 64 == 0 && a.out_ld * 2 == a.W.rows;
+}
+
+template <int EPI, bool HM, bool TAIL>
+static void pf_gemm_go(const pf_gemm_args& a, hipStream_t s) {
+    // 16 positions per wave when 32 would leave fewer than two waves per SIMD
+    const unsigned gx = (unsigned)((a.W.rows + 63) / 64), gy = (unsigned)((a.n + 63) / 64);
+    if ((size_t)gx * gy * 4 < 2048)
+        hipLaunchKernelGGL((k_pf_gemm_lds<EPI, HM, PF_KC, 16, TAIL>), dim3(gx, (unsigned)((a.n + 31) / 32)), dim3(256), 0, s, a);
+    else
+        hipLaunchKernelGGL((k_pf_gemm_lds<EPI, HM, PF_KC, 32, TAIL>), dim3(gx, gy), dim3(256), 0, s, a);
 }
 
 hipError_t launch_pf_gemm(int epi, const pf_gemm_args& a, hipStream_t s) {
-    if (a.n < 1 || a.W.rows % 8 || (epi == EPI_SWIGLU && a.W.rows % 16)) return hipErrorInvalidValue;
+    if (a.n < 1 || a.W.nb < 1 || a.W.rows % 8 || (epi == EPI_SWIGLU && a.W.rows % 16)) return hipErrorInvalidValue;
+    if (epi != EPI_SWIGLU && epi != EPI_STORE) return hipErrorInvalidValue;
     if (a.outc.q && (epi != EPI_SWIGLU || !a.outc.d || !a.outc.s || !pf_swiglu_cut_takes(a))) return hipErrorInvalidValue;
-    const dim3 grid((a.W.rows + 63) / 64, (a.n + 63) / 64);
-    const bool hm = a.W.mins != nullptr;   // Q4_1 table
-    if (a.W.nb % PF_KC == 0 && !getenv_pf_plain()) {
-        // 16 positions per wave when 32 would leave fewer than two waves per SIMD
-        const bool narrow = (size_t)grid.x * grid.y * 4 < 2048;
-        const dim3 g16(grid.x, (a.n + 31) / 32);
-#define SH_PF_LDS(EPI_, HM_)                                                                                      \
-    if (narrow) hipLaunchKernelGGL((k_pf_gemm_lds<EPI_, HM_, PF_KC, 16>), g16, dim3(256), 0, s, a);            \
-    else hipLaunchKernelGGL((k_pf_gemm_lds<EPI_, HM_, PF_KC, 32>), grid, dim3(256), 0, s, a);
-        if (epi == EPI_SWIGLU && hm) { SH_PF_LDS(EPI_SWIGLU, true) }
-        else if (epi == EPI_SWIGLU) { SH_PF_LDS(EPI_SWIGLU, false) }
-        else if (epi == EPI_STORE && hm) { SH_PF_LDS(EPI_STORE, true) }
-        else if (epi == EPI_STORE) { SH_PF_LDS(EPI_STORE, false) }
-        else return hipErrorInvalidValue;
-#undef SH_PF_LDS
-        return hipGetLastError();
+    const bool hm = a.W.mins != nullptr, tail = a.W.nb % PF_KC != 0;   // hm: Q4_1 table
+    if (epi == EPI_SWIGLU) {
+        if (hm) tail ? pf_gemm_go<EPI_SWIGLU, true, true>(a, s) : pf_gemm_go<EPI_SWIGLU, true, false>(a, s);
+        else tail ? pf_gemm_go<EPI_SWIGLU, false, true>(a, s) : pf_gemm_go<EPI_SWIGLU, false, false>(a, s);
+    } else {
+        if (hm) tail ? pf_gemm_go<EPI_STORE, true, true>(a, s) : pf_gemm_go<EPI_STORE, true, false>(a, s);
+        else tail ? pf_gemm_go<EPI_STORE, false, true>(a, s) : pf_gemm_go<EPI_STORE, false, false>(a, s);
     }
-    if (epi == EPI_SWIGLU && hm)
-        hipLaunchKernelGGL((k_pf_gemm<EPI_SWIGLU, true>), grid, dim3(256), 0, s, a);
-    else if (epi == EPI_SWIGLU)
-        hipLaunchKernelGGL((k_pf_gemm<EPI_SWIGLU, false>), grid, dim3(256), 0, s, a);
-    else if (epi == EPI_STORE && hm)
-        hipLaunchKernelGGL((k_pf_gemm<EPI_STORE, true>), grid, dim3(256), 0, s, a);
-    else if (epi == EPI_STORE)
-        hipLaunchKernelGGL((k_pf_gemm<EPI_STORE, false>), grid, dim3(256), 0, s, a);
-    else
-        return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

@@ -39,6 +39,21 @@ def test_gemm_matches_batch_kernel(rows, cols, n):
         assert same(y[i], t.gemv(x[i]))
 
 
+@pytest.mark.parametrize("rows,cols,n", [(8, 32, 1), (64, 96, 33), (72, 160, 64), (1032, 288, 130), (2048, 2080, 448),
+                                         (16384, 224, 512)])
+def test_gemm_partial_last_chunk(rows, cols, n):
+    """Block counts that are no multiple of the product's 4-block chunk (1, 3, 5, 9, 65 and 7 blocks), both wave tiles."""
+    import nunchi_amd
+    import oracle
+    raw = q4_random(rows, cols, rows + cols + n)
+    x = np.random.default_rng(n).standard_normal((n, cols)).astype(np.float32)
+    ctx = nunchi_amd.Context()
+    y = nunchi_amd.Q4Table(ctx, raw, rows, cols).gemm(x)
+    o = oracle.Q4Table(raw, rows, cols)
+    want = np.concatenate([o.gemv_batch(x[i:i + 64]) for i in range(0, n, 64)])
+    assert same(y, want), f"rel {rel(y, want):.2e}"
+
+
 def _prompt(n, vocab, seed):
     return np.random.default_rng(seed).integers(0, vocab, size=n).astype(np.int32)
 
@@ -115,6 +130,25 @@ def test_prefill_head_groups_and_windows(model_dir, E, heads, D, window):
                              swa_layers=(1,) if window else ())
     path = synth.cached("brain", shape, 21, model_dir)
     _check_batch(path, tokens=_prompt(45, 1000, 22), pre=_prompt(3, 1000, 23))
+
+
+def test_prefill_partial_last_chunk(model_dir):
+    """FFN down tables of 17 blocks, against the oracle; then every table but the o table's input 9 blocks wide (the
+    SwiGLU product and its cut among them), against single steps (attention narrower than n_embd, where imi's batch
+    differs from its own steps)."""
+    import nunchi_amd
+    from nunchi_amd import synth
+    kw = dict(n_layer=2, attn_layers=(1,), n_head=8, n_head_kv=4, head_dim=32, n_ff=544, n_vocab=1000)
+    _check_batch(synth.cached("brain", synth.BrainShape(n_embd=256, **kw), 25, model_dir), tokens=_prompt(45, 1000, 26),
+                 pre=_prompt(2, 1000, 27))
+    g = nunchi_amd.Brain(synth.cached("brain", synth.BrainShape(n_embd=288, **kw), 25, model_dir), n_ctx=64)
+    toks = _prompt(45, 1000, 26)
+    _, lg, _, ha = g.step_batch(toks, want_logits=True, hidden_all=True)
+    s = g.new_state()
+    for p, tok in enumerate(toks):
+        hp, lp, _ = g.step(int(tok), st=s)
+        assert same(hp, ha[p]), f"position {p}: batch and single step differ"
+    assert same(lg, lp)
 
 
 def test_prefill_attention_valu_form(tiny_model, monkeypatch):
