@@ -28,6 +28,38 @@ __device__ __forceinline__ void position_scales(const vtab_args& a, float* scl) 
     }
 }
 
+// rms_scale_wave's values by a half-wave (lane P of the half runs chain P; the same combine) over a row of 32 NT values in
+// memory, every operand requested first; in every lane of the half
+template <int NT>
+__device__ __forceinline__ float rms_scale_half_g(const float* x, float eps) {
+    const int hl = threadIdx.x & 31, base = threadIdx.x & 32;
+    float v[NT], a = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NT; t++) v[t] = x[32 * t + hl];
+#pragma unroll
+    for (int t = 0; t < NT; t++) a = fmaf(v[t], v[t], a);
+    auto at = [&](float f, int l) { return __shfl(f, base + (l & 31)); };
+    const float u = (a + at(a, hl + 8)) + (at(a, hl + 16) + at(a, hl + 24));   // lanes 0..7 of the half
+    const float r = u + at(u, hl + 4);
+    const float q = r + at(r, hl + 2);
+    const float s = at(q, 0) + at(q, 1);
+    return 1.0f / sqrtf(s / (float)(32 * NT) + eps);
+}
+
+// position_scales with a half-wave per row for the widths the scaled-order tables have (the four waves' eight rows at once)
+template <int P>
+__device__ __forceinline__ void position_scales_half(const vtab_args& a, float* scl) {
+    if (a.W.cols != 512 && a.W.cols != 1024) {
+        position_scales<P>(a, scl);
+        return;
+    }
+    for (int p = threadIdx.x >> 5; p < P; p += VX_THREADS / 32) {
+        const float* row = a.src + (size_t)p * a.src_ld;
+        const float s = a.W.cols == 512 ? rms_scale_half_g<16>(row, a.eps) : rms_scale_half_g<32>(row, a.eps);
+        if ((threadIdx.x & 31) == 0) scl[p] = s;
+    }
+}
+
 // columns [1024 q, 1024 q + 32 nbc) of the P positions, k-major: xs[block][column in block][position]
 // (imi/core/voice.cpp:157-166: the transposed input, normed first when the table follows a norm)
 // Thread t stages columns 4t..4t+3 of every position: all P 16-byte loads are in flight before the first LDS store
@@ -244,14 +276,21 @@ __global__ __launch_bounds__(VX_THREADS) void k_vtab_fold(vtab_args a) {
     table_epilogue<P, EPI, 8>(a, g0, acc, ev, et);
 }
 
-// scaled order (imi/core/tables.cpp:324-365, P = 12 or 6): thread (row, position) runs one chain over all columns
-// of fma(float(w) * d, x, acc); two row groups (16 rows) per workgroup. The workgroup stages 256 columns at a time,
-// one chunk ahead: each thread loads one 16-byte word of codes (16 columns of one row's block) and the block's scale
-// and stores the 16 products float(w) * d (exact: an int8 times an fp16 has at most 19 significant bits) to LDS, and
-// the positions' inputs (normed first for a VP_NORM table) go position-major beside them; a chain step then reads
-// 4 columns of its row and 4 of its position as one 16-byte LDS word each.
+// scaled order (imi/core/tables.cpp:324-365, P = 12 or 6): one chain per (row, position) over all columns of
+// fma(float(w) * d, x, acc); two row groups (16 rows) per workgroup, which are one 16 x 16 tile of
+// v_mfma_f32_16x16x4_f32 (positions past P repeat the last one and are dropped): its four K steps are four fused
+// multiply-adds in column order, each rounded once, bit for bit the VALU's chain, at 8 cycles a column where a dependent
+// VALU chain with its LDS reads ran at 15. A fifth wave runs the chains while the other four stage; its lane l supplies row / position l % 16, column l / 16 of
+// a step, and holds rows 4 (l / 16) + i of position l % 16. The workgroup stages 256 columns at a time, one chunk
+// ahead, requested one more chunk before that: each thread loads one 16-byte word of codes (16 columns of one row's block) and the block's scale and stores the
+// 16 products float(w) * d (exact: an int8 times an fp16 has at most 19 significant bits) to LDS, and the positions'
+// inputs (normed first for a VP_NORM table) beside them. Within each 16 columns LDS holds column 4 s + k at 4 k + s, so
+// a lane's four steps are one 16-byte word each.
+// Against a thread per chain: 512 columns 8.2 -> 6.0 us a launch (norm in front), 2048 columns 16 -> 13.3, 4096 at 12
+// positions 22.1; bound by the chains' dependent products (33 cycles a step) and, at 512 columns, by the launch, the norm's
+// own chain and the first chunk's way in.
 template <int P, int PRO, int EPI>
-__global__ __launch_bounds__(VX_THREADS) void k_vtab_scaled(vtab_args a) {
+__global__ __launch_bounds__(VX_THREADS + 64) void k_vtab_scaled(vtab_args a) {
     const uint64_t et = EPI == VE_SWIGLU ? kExp2Tab[threadIdx.x & 31] : 0;   // (first: its wait needs nothing later)
     constexpr int WC = 256, WS = WC + 4, NBK = WC / 32;   // columns per chunk, LDS row stride, blocks per chunk
     constexpr int NXQ = (P * (WC / 4) + VX_THREADS - 1) / VX_THREADS;   // input 16-byte words per thread per chunk
@@ -260,18 +299,17 @@ __global__ __launch_bounds__(VX_THREADS) void k_vtab_scaled(vtab_args a) {
     __shared__ __attribute__((aligned(16))) float sX[2][P * WS];
     __shared__ float scl[VX_MAX_P];
     __shared__ float ev[16 * VX_MAX_P];
-    const int t = threadIdx.x, rl = t / P, c = t - rl * P;
+    __shared__ float rs[16 * P];
+    const int t = threadIdx.x;
     const int nb = a.W.nb, K = a.W.cols, ng = a.W.rows_pad / 8, nch = (K + WC - 1) / WC, g0 = blockIdx.x * 2;
     // staging role: group gg, block jb of the chunk, row r8 of the group, half h of the block's 32 codes
     const int gg = t >> 7, jb = (t >> 4) & 7, r8 = (t >> 1) & 7, h = t & 1;
     const int grp = min(g0 + gg, ng - 1);   // (a workgroup's second group past the table reads the last one; dropped)
-    if (PRO == VP_NORM) {
-        position_scales<P>(a, scl);
-        __syncthreads();
-    }
+    const bool chain = t >= VX_THREADS;   // the last wave
     u32x4 gq;
     uint16_t gs;
-    f32x4 gx[NXQ];
+    f32x4 gx[NXQ], gn{};   // (gn: the norm weights of this thread's columns, the same four for every position)
+    static_assert(VX_THREADS % (WC / 4) == 0, "a thread stages the same columns of each of its positions");
     auto fetch = [&](int q) {   // every load unconditional, indices clamped into the buffers
         const int j = min(q * NBK + jb, nb - 1);
         const size_t blk = ((size_t)grp * nb + j) * 8 + r8;
@@ -282,6 +320,7 @@ __global__ __launch_bounds__(VX_THREADS) void k_vtab_scaled(vtab_args a) {
             const int idx = min(t + VX_THREADS * s, P * (WC / 4) - 1), p = idx / (WC / 4), k = min(q * WC + 4 * (idx % (WC / 4)), K - 4);
             gx[s] = *reinterpret_cast<const f32x4*>(a.src + (size_t)p * a.src_ld + k);
         }
+        if (PRO == VP_NORM) gn = *reinterpret_cast<const f32x4*>(a.norm_w + min(q * WC + 4 * (t % (WC / 4)), K - 4));
     };
     auto stash = [&](int b, int q) {
         const bool ok = q * NBK + jb < nb;   // a block past the table's columns stores zeros (never read)
@@ -291,10 +330,10 @@ __global__ __launch_bounds__(VX_THREADS) void k_vtab_scaled(vtab_args a) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             f32x4 o;
-            o.x = ok ? (float)(int)(signed char)(wv[i] & 0xFFu) * d : 0.0f;
-            o.y = ok ? (float)(int)(signed char)((wv[i] >> 8) & 0xFFu) * d : 0.0f;
-            o.z = ok ? (float)(int)(signed char)((wv[i] >> 16) & 0xFFu) * d : 0.0f;
-            o.w = ok ? (float)(int)(signed char)(wv[i] >> 24) * d : 0.0f;
+            o.x = ok ? (float)(int)(signed char)((wv[0] >> (8 * i)) & 0xFFu) * d : 0.0f;
+            o.y = ok ? (float)(int)(signed char)((wv[1] >> (8 * i)) & 0xFFu) * d : 0.0f;
+            o.z = ok ? (float)(int)(signed char)((wv[2] >> (8 * i)) & 0xFFu) * d : 0.0f;
+            o.w = ok ? (float)(int)(signed char)((wv[3] >> (8 * i)) & 0xFFu) * d : 0.0f;
             *reinterpret_cast<f32x4*>(dst + 4 * i) = o;
         }
 #pragma unroll
@@ -304,36 +343,72 @@ __global__ __launch_bounds__(VX_THREADS) void k_vtab_scaled(vtab_args a) {
                 const int p = idx / (WC / 4), k4 = idx % (WC / 4), col = q * WC + 4 * k4;
                 f32x4 e = gx[s];
                 if (PRO == VP_NORM && col < K) {
-                    const f32x4 nw = *reinterpret_cast<const f32x4*>(a.norm_w + col);
-                    e.x = e.x * scl[p] * nw.x; e.y = e.y * scl[p] * nw.y;
-                    e.z = e.z * scl[p] * nw.z; e.w = e.w * scl[p] * nw.w;
+                    e.x = e.x * scl[p] * gn.x; e.y = e.y * scl[p] * gn.y;
+                    e.z = e.z * scl[p] * gn.z; e.w = e.w * scl[p] * gn.w;
                 }
-                *reinterpret_cast<f32x4*>(&sX[b][p * WS + 4 * k4]) = e;
+                float* xd = &sX[b][p * WS + 16 * (k4 >> 2) + (k4 & 3)];
+                xd[0] = e.x;
+                xd[4] = e.y;
+                xd[8] = e.z;
+                xd[12] = e.w;
             }
         }
     };
-    fetch(0);
-    stash(0, 0);
+    if (!chain) {   // (the first chunk requested before the norm scales)
+        fetch(0);
+        if (PRO == VP_NORM) position_scales_half<P>(a, scl);
+    }
+    if (PRO == VP_NORM) __syncthreads();
+    if (!chain) {
+        stash(0, 0);
+        if (nch > 1) fetch(1);
+    }
     __syncthreads();
-    float acc = 0.0f;
-    const bool live = t < 16 * P;
-    const int rr = live ? rl : 0, cc = live ? c : 0;
+    const int li = t & 15, lq = (t & 63) >> 4;
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int q = 0; q < nch; q++) {
-        const int b = q & 1, nk4 = min(WC, K - q * WC) / 4;
-        if (q + 1 < nch) fetch(q + 1);
-        const float* wrow = &sW[b][rr * WS];
-        const float* xrow = &sX[b][cc * WS];
-        for (int k4 = 0; k4 < nk4; k4++) {
-            const f32x4 w = *reinterpret_cast<const f32x4*>(wrow + 4 * k4);
-            const f32x4 x = *reinterpret_cast<const f32x4*>(xrow + 4 * k4);
-            acc = fmaf(w.x, x.x, acc);
-            acc = fmaf(w.y, x.y, acc);
-            acc = fmaf(w.z, x.z, acc);
-            acc = fmaf(w.w, x.w, acc);
+        const int b = q & 1, n32 = min(WC, K - q * WC) / 32;
+        if (!chain) {
+            if (q + 1 < nch) stash(b ^ 1, q + 1);
+            if (q + 2 < nch) fetch(q + 2);   // (two chunks ahead: a whole chunk's chains to arrive in)
+        } else {   // 32 columns (8 steps) at a time, the next ones' operands read first
+            const float* wr = &sW[b][li * WS + 4 * lq];
+            const float* xr = &sX[b][min(li, P - 1) * WS + 4 * lq];
+            f32x4 w[2][2], x[2][2];
+            auto read = [&](int z, int g) {
+#pragma unroll
+                for (int u = 0; u < 2; u++) {
+                    w[z][u] = *reinterpret_cast<const f32x4*>(wr + 32 * g + 16 * u);
+                    x[z][u] = *reinterpret_cast<const f32x4*>(xr + 32 * g + 16 * u);
+                }
+            };
+            auto run = [&](int z) {
+#pragma unroll
+                for (int s = 0; s < 8; s++) o = __builtin_amdgcn_mfma_f32_16x16x4f32(w[z][s >> 2][s & 3], x[z][s >> 2][s & 3], o, 0, 0, 0);
+            };
+            read(0, 0);
+            if (n32 == NBK) {   // (whole chunks with static registers: moves between sets hold up the next product)
+#pragma unroll
+                for (int g = 0; g < NBK; g++) {
+                    if (g + 1 < NBK) read((g + 1) & 1, g + 1);
+                    run(g & 1);
+                }
+            } else {
+                for (int g = 0; g < n32; g++) {
+                    run(0);
+                    if (g + 1 < n32) read(0, g + 1);
+                }
+            }
         }
-        if (q + 1 < nch) stash(b ^ 1, q + 1);
         __syncthreads();
     }
+    // the epilogue's thread per (row, position) takes its result from LDS
+    if (chain && li < P) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) rs[(4 * lq + i) * P + li] = o[i];
+    }
+    __syncthreads();
+    const float acc = t < 16 * P ? rs[t] : 0.0f;
     table_epilogue<P, EPI, 16>(a, g0, acc, ev, et);
 }
 
@@ -566,7 +641,7 @@ __global__ __launch_bounds__(256) void k_vsample(vsample_args a) {
 template <int P, int PRO, int EPI>
 hipError_t launch_vtab_p(const vtab_args& a, hipStream_t s) {
     if constexpr (P == 6 || P == 12)
-        hipLaunchKernelGGL((k_vtab_scaled<P, PRO, EPI>), dim3(a.units), dim3(VX_THREADS), 0, s, a);
+        hipLaunchKernelGGL((k_vtab_scaled<P, PRO, EPI>), dim3(a.units), dim3(VX_THREADS + 64), 0, s, a);
     else {
         if constexpr (EPI != VE_SWIGLU) {
             if (a.part && a.W.nb > VX_NJ) {

@@ -70,6 +70,15 @@ def test_codebook_counts(model_dir, n_cb, schedule):
     _play(path, n_cb, schedule, n_frames=1)
 
 
+@pytest.mark.parametrize("n_cb,E,n_ff", [(12, 288, 800), (6, 512, 288), (12, 1024, 2080), (6, 96, 32)])
+def test_scaled_order_widths(model_dir, n_cb, E, n_ff):
+    """The scaled order's tables at widths that end inside a 256-column chunk (and are narrower than one), and the norm
+    scales' half-wave widths (512 and 1024)."""
+    from nunchi_amd import synth
+    path = synth.cached("voice", _shape(n_cb=n_cb, n_embd=E, n_ff=n_ff, n_layer=1, n_vocab=96), 10, model_dir)
+    _play(path, n_cb + E, (n_cb // 2, n_cb // 2), n_frames=1)
+
+
 def test_narrow_heads_and_odd_groups(model_dir):
     """head_dim 32, 4 query heads per kv head, widths that are not powers of two, an odd number of qkvg row groups."""
     from nunchi_amd import synth
