@@ -85,10 +85,11 @@ __device__ __forceinline__ float wval(const wraw<F32W>& r, int s) {   // (s know
 // load costs its wave about as many cycles as one of these products), requested DC chunks of 32 columns ahead. Every
 // global load is unconditional (chunk indices clamped; past the table's last column nothing is multiplied), so the
 // compiler's wait counts stay exact.
-// At 384 positions: b|c|x 2304 x 768 33.0 -> 21.3 us, gate|up 4096 x 768 44.7 -> 30.2, down 768 x 2048 48 -> 37, the
-// 4096-wide pre_encode 90.7 -> 48.0; at 29 positions gate|up 12.6 -> 9.4, down 25 -> 16.6 (with feature-major inputs read
-// a word per step: 28.0, 44.0 and 65.3 for the first, second and fourth, 24.6 for the last). Bound by the vector loads
-// (3 KB per 32 columns and 16 x 16 outputs), then by the chains' 8 cycles a column.
+// At 384 positions, against one column per v_mfma_f32_4x4x1_16b_f32: b|c|x 2304 x 768 33.0 -> 21.2 us, gate|up 4096 x 768
+// 44.7 -> 30.0, o and down (768 x 768, 768 x 2048) 33.7 -> 19.3 on average, mlp.3 2048 x 2048 63.6 -> 37.4, pre_encode
+// 768 x 4096 90.7 -> 47.3. (With this product but feature-major inputs, read a word per step: 28.0, 44.0, 33.4, 51.3 and
+// 65.3; at 29 positions gate|up 12.6 and down 24.6 against 9.4 and 16.6.) Bound by the vector loads (3 KB per 32 columns
+// and 16 x 16 outputs), then by the chains' 8 cycles a column.
 template <int EPI, bool F32W, int MP>
 __global__ __launch_bounds__(ET) void k_etab(etab_args a) {
     typedef float v4f __attribute__((ext_vector_type(4)));
