@@ -165,23 +165,25 @@ __global__ __launch_bounds__(256) void k_pf_cut(pf_cutk_args a) {
 // position), block by block in order: acc = fma(float(isum), d * dx, acc), cor = fma(d, s, cor), and at the end
 // out = fma(-8, cor, acc) (imi/core/tables.cpp:419-454, the batch kernel imi's prefill uses); Q4_1 tables take the
 // block minimum m in the cor chain and end as acc + cor.
-// Per workgroup the operands of KC blocks
-// (64 rows of codes, their scales and, for Q4_1, minima; 64 positions of input codes and their (d, s)) are fetched
-// with wide coalesced loads into registers while the waves run the previous KC blocks from LDS, then stored to the
-// other half of a double buffer, the codes already split into their low and high nibbles. Two of the three fp32 operations per (row, position, block) run on
-// the matrix cores as K = 1 outer products, v_mfma_f32_16x16x1_4b_f32, whose four 16 x 16 blocks are the wave's
-// (row tile, position tile) pairs: dd = d x dx (accumulator 0) and cor = fma(d, s, cor) (the running cor as the
-// accumulator, one product per block in block order). That operation rounds once, like fmaf: it equals the VALU's
-// fmaf bit for bit, denormals and the fused cancellation included (measured on 4.2 M cases); d x dx + 0 differs from
-// the product only in the sign of a zero, which the acc chain (started at +0) cannot see. Only acc =
-// fma(float(isum), dd, acc) stays on the VALU. A workgroup is 4 waves over 64 rows x 2 PW positions, a wave 32 rows x
-// PW positions: PW = 32 for tables with enough rows, 16 for the narrow ones (2048 rows: two waves per SIMD instead of
-// one), whose matrix-core blocks for the missing position tile are computed on a repeated position and dropped.
-// TAIL: block counts that are no multiple of KC. The last chunk's missing blocks re-read the last block and are staged
-// with zero codes and scales, which add +0 to chains that are never -0; the clamps cost the whole chunks' path about 3 %
-// (16384 x 2048 at 448 positions 74.9 -> 77.1 us), so that one is compiled without them. Against an unstaged product of
-// the same wave tiles: 4096 x 2080 at 448 / 100 / 17 positions 42.9 / 23.8 / 22.0 -> 37.6 / 15.5 / 14.4 us, 1024 x 8160
-// at 64 79.5 -> 48.1, 16384 x 288 at 512 39.1 -> 33.4.
+// Per workgroup the operands of KC blocks (64 rows of codes, their scales and, for Q4_1, minima; 64 positions of input
+// codes and their (d, s)) are fetched with wide coalesced loads into registers while the waves run the previous KC blocks
+// from LDS, then stored to the other half of a double buffer, the codes already split into their low and high nibbles.
+// Two of the three fp32 operations per (row, position, block) run on the matrix cores as K = 1 outer products,
+// v_mfma_f32_16x16x1_4b_f32, whose four 16 x 16 blocks are the wave's (row tile, position tile) pairs: dd = d x dx
+// (accumulator 0) and cor = fma(d, s, cor) (the running cor as the accumulator, one product per block in block order).
+// That operation rounds once, like fmaf: it equals the VALU's fmaf bit for bit, denormals and the fused cancellation
+// included (measured on 4.2 M cases); d x dx + 0 differs from the product only in the sign of a zero, which the acc chain
+// (started at +0) cannot see. Only acc = fma(float(isum), dd, acc) stays on the VALU. A workgroup is 4 waves over 64 rows
+// x 2 PW positions, a wave 32 rows x PW positions: PW = 32 for tables with enough rows, 16 for the narrow ones (2048
+// rows: two waves per SIMD instead of one), whose matrix-core blocks for the missing position tile are computed on a
+// repeated position and dropped.
+// TAIL: block counts that are no multiple of KC. The last chunk's missing blocks are staged as the last block again and
+// not multiplied (multiplied with zero codes and scales they would make a NaN of an infinite (d, s)): the wide tile's
+// block loop ends early, the narrow one, whose unrolled body would lose its interleaving by that (8192 x 8160 at 64
+// positions 55.8 -> 59.4 us), runs the last blocks one by one. The clamps cost the whole chunks' path about 3 % (16384 x
+// 2048 at 448 positions 74.9 -> 77.1 us), so that one is compiled without them. Against an unstaged product of the same
+// wave tiles, input cut and launches included: 4096 x 2080 at 448 / 100 / 17 positions 48.1 / 34.1 / 32.1 -> 41.1 / 21.5 /
+// 20.8 us, 1024 x 8160 at 64 105.8 -> 54.6, 16384 x 288 at 512 42.5 -> 34.1, 2048 x 32 at 17 9.8 -> 9.7.
 template <int EPI, bool HM, int KC, int PW, bool TAIL>
 __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_lds(pf_gemm_args a) {
     typedef float v16f __attribute__((ext_vector_type(16)));
@@ -241,12 +243,7 @@ __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_
             gxs[q] = px[q][xo + (ptrdiff_t)sdo];
         }   // (threads past P * KC re-read the last pair; they store nothing)
     };
-    auto stash = [&](int buf, int c) {
-        if (TAIL && c * KC + t % KC >= nb) {
-#pragma unroll
-            for (int q = 0; q < NA; q++) ga[q] = u32x4{0, 0, 0, 0};
-            gd = gm = u32x4{0, 0, 0, 0};
-        }
+    auto stash = [&](int buf) {
 #pragma unroll
         for (int q = 0; q < NA; q++) {   // byte k of the record: low nibble of code byte k (k < 16), high of k - 16
             const int idx = t + 256 * q;
@@ -286,45 +283,57 @@ __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_
     const int orow = rl + 16 * (lane >> 5) + li, opos = pl + 16 * (NTW == 2 ? (lane >> 4) & 1 : 0) + li;
     const uint64_t et = EPI == EPI_SWIGLU ? kExp2Tab[t & 31] : 0;   // (requested first: its wait needs nothing later)
     fetch(0);
-    stash(0, 0);
+    stash(0);
     if (EPI == EPI_SWIGLU && t < 32) sE[t] = et;
     __syncthreads();
-    for (int c = 0; c < nch; c++) {
+    // block jb of the chunk in half buf; acc in place, cor returned
+    auto block = [&](int buf, int jb, float (&acc)[16], v16f cor) -> v16f {
+        i32x4 isum[2][NTW];
+        long cb[NTW];
+#pragma unroll
+        for (int nt = 0; nt < NTW; nt++)   // (li & 8: the halves were swapped, which spreads the reads over the banks)
+            cb[nt] = ((const long*)&sB[buf][jb][pl + 16 * nt + li][0])[lq ^ ((li >> 3) << 1)];
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++) {   // columns 8 (lq & 1) .. + 7, low nibbles for lq < 2, else high
+            const long av = *(const long*)&sA[buf][(rl + 16 * mt + li) * SA + 8 * jb + 2 * lq];
+#pragma unroll
+            for (int nt = 0; nt < NTW; nt++)
+                isum[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, cb[nt], i32x4{0, 0, 0, 0}, 0, 0, 0);
+        }
+        const float dl = h2f(sD[buf][jb][orow]);
+        const float ml = HM ? h2f(sM[buf][jb][HM ? orow : 0]) : dl;
+        const float2 xl = sX[buf][jb][opos];
+        const v16f dd = __builtin_amdgcn_mfma_f32_16x16x1f32(dl, xl.x, zero, 0, 0, 0);
+        cor = __builtin_amdgcn_mfma_f32_16x16x1f32(ml, xl.y, cor, 0, 0, 0);
+#pragma unroll
+        for (int mt = 0; mt < 2; mt++)
+#pragma unroll
+            for (int nt = 0; nt < NTW; nt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int k = 4 * (2 * mt + nt) + i;
+                    acc[k] = fmaf((float)isum[mt][nt][i], dd[k], acc[k]);
+                }
+        return cor;
+    };
+    constexpr bool PEEL = TAIL && PW == 16;   // (the last chunk's blocks after the loop)
+    for (int c = 0; c < (PEEL ? nb / KC : nch); c++) {
         const int buf = c & 1;
         if (c + 1 < nch) fetch(c + 1);
         // the narrow tiles (fewer than 2 workgroups per CU) take a whole chunk's blocks in one unrolled body, their
         // LDS reads and matrix-core products all issued ahead of the chains (the register room 2 workgroups per CU allow)
 #pragma unroll(PW == 16 ? KC : 2)
         for (int jb = 0; jb < KC; jb++) {
-            i32x4 isum[2][NTW];
-            long cb[NTW];
-#pragma unroll
-            for (int nt = 0; nt < NTW; nt++)   // (li & 8: the halves were swapped, which spreads the reads over the banks)
-                cb[nt] = ((const long*)&sB[buf][jb][pl + 16 * nt + li][0])[lq ^ ((li >> 3) << 1)];
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++) {   // columns 8 (lq & 1) .. + 7, low nibbles for lq < 2, else high
-                const long av = *(const long*)&sA[buf][(rl + 16 * mt + li) * SA + 8 * jb + 2 * lq];
-#pragma unroll
-                for (int nt = 0; nt < NTW; nt++)
-                    isum[mt][nt] = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, cb[nt], i32x4{0, 0, 0, 0}, 0, 0, 0);
-            }
-            const float dl = h2f(sD[buf][jb][orow]);
-            const float ml = HM ? h2f(sM[buf][jb][HM ? orow : 0]) : dl;
-            const float2 xl = sX[buf][jb][opos];
-            const v16f dd = __builtin_amdgcn_mfma_f32_16x16x1f32(dl, xl.x, zero, 0, 0, 0);
-            cor = __builtin_amdgcn_mfma_f32_16x16x1f32(ml, xl.y, cor, 0, 0, 0);
-#pragma unroll
-            for (int mt = 0; mt < 2; mt++)
-#pragma unroll
-                for (int nt = 0; nt < NTW; nt++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int k = 4 * (2 * mt + nt) + i;
-                        acc[k] = fmaf((float)isum[mt][nt][i], dd[k], acc[k]);
-                    }
+            if (TAIL && !PEEL && c * KC + jb >= nb) break;
+            cor = block(buf, jb, acc, cor);
         }
-        if (c + 1 < nch) stash(buf ^ 1, c + 1);
+        if (c + 1 < nch) stash(buf ^ 1);
         __syncthreads();
+    }
+    if (PEEL) {
+#pragma unroll 1
+        for (int jb = 0; jb < nb % KC; jb++) cor = block((nb / KC) & 1, jb, acc, cor);
+        if (EPI == EPI_SWIGLU) __syncthreads();   // (the cut below reuses the code tiles' space)
     }
     const int rbase = r0 + rl, pbase = p0 + pl;
     // EPI_SWIGLU with outc: the workgroup's 64 rows are one 32-channel cut block of the output; its activations are

@@ -54,6 +54,25 @@ def test_gemm_partial_last_chunk(rows, cols, n):
     assert same(y, want), f"rel {rel(y, want):.2e}"
 
 
+@pytest.mark.parametrize("rows,nb,n", [(8, 1, 2), (72, 5, 17), (64, 6, 33), (16384, 7, 128)])
+@pytest.mark.parametrize("value", [2e37, -3e38])
+def test_gemm_partial_last_chunk_overflow(rows, nb, n, value):
+    """Finite inputs whose last block's scale times code sum overflows: the oracle's infinities (and NaNs, where its own
+    chains form them), not NaNs from the last chunk's missing blocks; position 0 stays finite. Both wave tiles."""
+    import nunchi_amd
+    import oracle
+    raw = q4_random(rows, 32 * nb, rows + nb)
+    x = np.random.default_rng(n).standard_normal((n, 32 * nb)).astype(np.float32)
+    x[1:, -32:] = value
+    y = nunchi_amd.Q4Table(nunchi_amd.Context(), raw, rows, 32 * nb).gemm(x)
+    o = oracle.Q4Table(raw, rows, 32 * nb)
+    want = np.concatenate([o.gemv_batch(x[i:i + 64]) for i in range(0, n, 64)])
+    assert np.isinf(want[1:]).any() and np.isfinite(want[0]).all()
+    assert np.array_equal(np.isnan(y), np.isnan(want))
+    k = ~np.isnan(want)
+    assert same(y[k], want[k])
+
+
 def _prompt(n, vocab, seed):
     return np.random.default_rng(seed).integers(0, vocab, size=n).astype(np.int32)
 
