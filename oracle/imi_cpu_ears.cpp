@@ -282,10 +282,15 @@ int ears::encode(const float* pcm, int n, std::vector<float>& out) {   // imi/co
     const int T2 = (n_fr + 1) / 2, F2 = n_mel / 2, T4 = (T2 + 1) / 2, F4 = F2 / 2, P = (T4 + 1) / 2, F8 = F4 / 2;
     const int C = n_ch, E = n_embd;
     auto ch12 = [](int v) { return (size_t)(v + 11) / 12 * 12; };
-    xt.resize(std::max({ch12(T4 * F4) * C, ch12(P * F8) * C, ch12(P) * pre.cols, ch12(P) * n_ff, ch12(P) * n_out,
-                        ch12(P) * mlp1.rows}));
-    buf.resize(std::max({(size_t)T2 * F2 * C, (size_t)T4 * F4 * C, (size_t)P * layers[0].in.rows, (size_t)P * 3 * E,
-                         (size_t)P * n_ff, (size_t)P * n_out, (size_t)P * mlp1.rows}));
+    int in_rows = 0, in_cols = E;   // (the widest layer tables' rows and inputs)
+    for (const layer& L : layers) {
+        in_rows = std::max(in_rows, L.in.rows);
+        in_cols = std::max(in_cols, L.out.cols);
+    }
+    xt.resize(std::max({ch12(T4 * F4) * C, ch12(P * F8) * C, ch12(P) * pre.cols, ch12(P) * in_cols, ch12(P) * n_ff,
+                        ch12(P) * n_out, ch12(P) * mlp1.rows}));
+    buf.resize(std::max({(size_t)T2 * F2 * C, (size_t)T4 * F4 * C, (size_t)P * in_rows, (size_t)P * n_ff,
+                         (size_t)P * n_out, (size_t)P * mlp1.rows}));
     buf2.resize((size_t)T4 * F4 * C);
     xres.resize((size_t)P * E);
 

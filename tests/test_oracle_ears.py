@@ -70,6 +70,19 @@ def test_threads_do_not_change_the_rows(tiny_ears):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize("kw", [dict(n_embd=768, n_head=3, head_dim=32, layers="c"),
+                                dict(n_embd=96, n_head=32, head_dim=128, layers="ca")])
+def test_layers_wider_than_the_ffn(model_dir, kw):
+    """A width, and an attention, wider than the FFN, the projector and the downsampler's features."""
+    from nunchi_amd import synth
+    shape = synth.EarsShape(n_mel=24, n_ch=8, n_ff=40, n_head_kv=1, window=5, n_out=8, **kw)
+    path = synth.cached("ears", shape, 4, model_dir)
+    pcm = synth.clip(37123, 8)
+    out = oracle.Ears(path, threads=4).encode(pcm)
+    truth, _ = exact.ears(path, pcm)
+    assert oracle.rel(out, truth) < TOL
+
+
 def test_short_clips(tiny_ears):
     """Clips shorter than one 400-sample frame still give one frame and one position (ears.cpp:203)."""
     from nunchi_amd import synth
