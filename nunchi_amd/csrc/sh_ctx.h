@@ -117,7 +117,8 @@ struct sh_ctx {
     bool use_graphs = true;
     // prefill work buffers (PF_MAX_N positions, made on first use)
     char* pf_mem = nullptr;
-    float *pf_x = nullptr, *pf_y = nullptr, *pf_big = nullptr, *pf_act = nullptr, *pf_hid = nullptr;
+    float *pf_x = nullptr, *pf_y = nullptr, *pf_big = nullptr, *pf_hid = nullptr;
+    char* pf_act = nullptr;           // the FFN activations, cut
     int8_t* pf_q = nullptr;
     float *pf_d = nullptr, *pf_s = nullptr, *pf_emb = nullptr;
     int32_t* pf_tok = nullptr;

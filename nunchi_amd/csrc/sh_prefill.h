@@ -53,9 +53,9 @@ struct pf_gemm_args {
     q4dev W;
     int n;
     pf_cut in;              // the input, cut (W.nb blocks)
-    float* out;             // EPI_STORE: [n][out_ld] rows of W; EPI_SWIGLU: [n][out_ld] silu(gate) * up channels
-    int out_ld;
-    pf_cut outc;            // EPI_SWIGLU with outc.q set: the channels cut (out_ld / 32 blocks) instead of stored
+    float* out;             // EPI_STORE: [n][out_ld] rows of W
+    int out_ld;             // EPI_SWIGLU: the silu(gate) * up channels, W.rows / 2 (a multiple of 32)
+    pf_cut outc;            // EPI_SWIGLU: the channels, cut (out_ld / 32 blocks)
 };
 
 struct pf_cutk_args {       // cut of n rows of K floats
@@ -80,9 +80,6 @@ struct pf_attn_args {       // causal attention of n positions (keys and values 
 
 hipError_t launch_pf_rows(int mode, const pf_rows_args& a, hipStream_t s);
 hipError_t launch_pf_gemm(int epi, const pf_gemm_args& a, hipStream_t s);
-// whether launch_pf_gemm takes EPI_SWIGLU with the cut output for these arguments (the staged kernel, whole 64-row
-// workgroups, each one 32-channel block)
-bool pf_swiglu_cut_takes(const pf_gemm_args& a);
 hipError_t launch_pf_cut(const pf_cutk_args& a, hipStream_t s);
 // the conv along positions and its cut; the conv memory update rides on the next launch_pf_rows (its conv field)
 hipError_t launch_pf_conv_lanes(const pf_conv_args& a, hipStream_t s);

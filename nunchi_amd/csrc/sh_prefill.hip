@@ -336,9 +336,8 @@ __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_
         if (EPI == EPI_SWIGLU) __syncthreads();   // (the cut below reuses the code tiles' space)
     }
     const int rbase = r0 + rl, pbase = p0 + pl;
-    // EPI_SWIGLU with outc: the workgroup's 64 rows are one 32-channel cut block of the output; its activations are
-    // staged in LDS (the code tiles' space, free after the last chunk's barrier), [position][channel], 33 floats apart
-    const bool cut_out = EPI == EPI_SWIGLU && a.outc.q != nullptr;
+    // EPI_SWIGLU: the workgroup's 64 rows are one 32-channel cut block of the output; its activations are staged in
+    // LDS (the code tiles' space, free after the last chunk's barrier), [position][channel], 33 floats apart
     float* act = reinterpret_cast<float*>(&sA[0][0]);
 #pragma unroll
     for (int mt = 0; mt < 2; mt++)
@@ -359,14 +358,8 @@ __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_
                 const float s0 = __shfl_xor(lo ? v[2] : v[0], 32), s1 = __shfl_xor(lo ? v[3] : v[1], 32);
                 const float g0 = lo ? v[0] : s0, g1 = lo ? v[1] : s1, u0 = lo ? s0 : v[2], u1 = lo ? s1 : v[3];
                 const int ch = (rl + 16 * mt) / 2 + 4 * (lq & 1) + (lo ? 0 : 2);   // channel within the workgroup's 32
-                if (cut_out) {   // to LDS for the block cut below
-                    act[(pl + 16 * nt + li) * 33 + ch] = silu_t(g0, sE) * u0;
-                    act[(pl + 16 * nt + li) * 33 + ch + 1] = silu_t(g1, sE) * u1;
-                } else if (p < n && rbase + 16 * mt < rows) {
-                    float* o = a.out + (size_t)p * a.out_ld + r0 / 2 + ch;
-                    o[0] = silu_t(g0, sE) * u0;
-                    o[1] = silu_t(g1, sE) * u1;
-                }
+                act[(pl + 16 * nt + li) * 33 + ch] = silu_t(g0, sE) * u0;   // to LDS for the block cut below
+                act[(pl + 16 * nt + li) * 33 + ch + 1] = silu_t(g1, sE) * u1;
             } else if (p < n) {
                 float* o = a.out + (size_t)p * a.out_ld + rr0;
 #pragma unroll
@@ -374,7 +367,7 @@ __global__ __launch_bounds__(256, (KC == 4 && PW == 32) ? 3 : 2) void k_pf_gemm_
                     if (rr0 + i < rows) o[i] = v[i];
             }
         }
-    if (EPI == EPI_SWIGLU && cut_out) {
+    if (EPI == EPI_SWIGLU) {
         // the cut of each position's block (imi_cut32's values, as cut_store): thread (position, quarter) holds 8
         // channels; amax and the code sum are order-free reductions, over the quad of lanes by DPP
         static_assert(sizeof(sA) >= (size_t)P * 33 * sizeof(float), "activation staging");
@@ -934,10 +927,6 @@ hipError_t launch_pf_rows(int mode, const pf_rows_args& a, hipStream_t s) {
 #define PF_KC 4   // blocks staged per step of the LDS-staged product
 #endif
 
-bool pf_swiglu_cut_takes(const pf_gemm_args& a) {
-    return a.n >= 1 && a.W.rows % 64 == 0 && a.out_ld * 2 == a.W.rows;
-}
-
 template <int EPI, bool HM, bool TAIL>
 static void pf_gemm_go(const pf_gemm_args& a, hipStream_t s) {
     // 16 positions per wave when 32 would leave fewer than two waves per SIMD
@@ -949,9 +938,11 @@ static void pf_gemm_go(const pf_gemm_args& a, hipStream_t s) {
 }
 
 hipError_t launch_pf_gemm(int epi, const pf_gemm_args& a, hipStream_t s) {
-    if (a.n < 1 || a.W.nb < 1 || a.W.rows % 8 || (epi == EPI_SWIGLU && a.W.rows % 16)) return hipErrorInvalidValue;
+    if (a.n < 1 || a.W.nb < 1 || a.W.rows % 8) return hipErrorInvalidValue;
     if (epi != EPI_SWIGLU && epi != EPI_STORE) return hipErrorInvalidValue;
-    if (a.outc.q && (epi != EPI_SWIGLU || !a.outc.d || !a.outc.s || !pf_swiglu_cut_takes(a))) return hipErrorInvalidValue;
+    // (SwiGLU: whole 64-row workgroups, each one 32-channel block of the cut)
+    if (epi == EPI_SWIGLU && (a.W.rows % 64 || a.out_ld * 2 != a.W.rows || !a.outc.q || !a.outc.d || !a.outc.s))
+        return hipErrorInvalidValue;
     const bool hm = a.W.mins != nullptr, tail = a.W.nb % PF_KC != 0;   // hm: Q4_1 table
     if (epi == EPI_SWIGLU) {
         if (hm) tail ? pf_gemm_go<EPI_SWIGLU, true, true>(a, s) : pf_gemm_go<EPI_SWIGLU, true, false>(a, s);

@@ -27,7 +27,7 @@ int prefill_buffers(sh_ctx* c) {
     const size_t big = std::max<size_t>(3 * E, c->nqkv), kmax = std::max<size_t>({E, (size_t)I.n_ff, Hq});
     size_t off = 0;
     auto room = [&](size_t bytes) { const size_t at = off; off += (bytes + 255) / 256 * 256; return at; };
-    const size_t o_x = room(N * E * 4), o_y = room(N * E * 4), o_big = room(N * big * 4), o_act = room(N * I.n_ff * 4);
+    const size_t o_x = room(N * E * 4), o_y = room(N * E * 4), o_big = room(N * big * 4), o_act = room(N * I.n_ff / 4 * 5);
     const size_t o_hid = room(N * E * 4), o_q = room(N * kmax), o_d = room(N * kmax / 32 * 4), o_s = room(N * kmax / 32 * 4);
     const size_t o_tok = room(N * 4), o_emb = room(N * E * 4);
     char* m = nullptr;
@@ -36,7 +36,7 @@ int prefill_buffers(sh_ctx* c) {
     c->pf_x = (float*)(m + o_x);
     c->pf_y = (float*)(m + o_y);
     c->pf_big = (float*)(m + o_big);
-    c->pf_act = (float*)(m + o_act);
+    c->pf_act = m + o_act;
     c->pf_hid = (float*)(m + o_hid);
     c->pf_q = (int8_t*)(m + o_q);
     c->pf_d = (float*)(m + o_d);
@@ -91,24 +91,24 @@ int enqueue_chunk(sh_ctx* c, sh_state* st, int m, bool have_tokens, bool have_em
     r.w_pre = c->layers[0].attn_norm;
     r.cut = cut;
     PCHK(launch_pf_rows(PFR_FIRST, r, s));
-    auto gemm = [&](const q4dev& W, int epi, float* out, int ld, const pf_cut& in) {
+    auto gemm = [&](const q4dev& W, float* out, int ld, const pf_cut& in) {
         pf_gemm_args g{};
         g.W = W;
         g.n = m;
         g.in = in;
         g.out = out;
         g.out_ld = ld;
-        return launch_pf_gemm(epi, g, s);
+        return launch_pf_gemm(EPI_STORE, g, s);
     };
-    // the FFN activations' cut, written by the gate|up products themselves into the activation buffer's space (their
-    // input cut is still being read meanwhile, so not the shared cut buffer)
+    // the FFN activations' cut, written by the gate|up products themselves (their input cut is still being read
+    // meanwhile, so not the shared cut buffer)
     const size_t nact = (size_t)PF_MAX_N * I.n_ff;
-    const pf_cut act_cut{(int8_t*)c->pf_act, (float*)((char*)c->pf_act + nact), (float*)((char*)c->pf_act + nact + nact / 8)};
+    const pf_cut act_cut{(int8_t*)c->pf_act, (float*)(c->pf_act + nact), (float*)(c->pf_act + nact + nact / 8)};
     for (size_t il = 0; il < c->layers.size(); il++) {
         const layer_dev& L = c->layers[il];
         pf_conv_args cv{};   // (a conv layer: its memory update rides on the next rows launch)
         if (L.conv) {
-            PCHK(gemm(L.in_proj, EPI_STORE, c->pf_big, 3 * E, cut));
+            PCHK(gemm(L.in_proj, c->pf_big, 3 * E, cut));
             cv.bcx = c->pf_big;
             cv.w = L.conv_w;
             cv.state = st->conv + (size_t)L.ci * I.d_conv * E;
@@ -117,9 +117,9 @@ int enqueue_chunk(sh_ctx* c, sh_state* st, int m, bool have_tokens, bool have_em
             cv.d_conv = I.d_conv;
             cv.cut = cut;
             PCHK(launch_pf_conv_lanes(cv, s));
-            PCHK(gemm(L.out_proj, EPI_STORE, c->pf_y, E, cut));
+            PCHK(gemm(L.out_proj, c->pf_y, E, cut));
         } else {
-            PCHK(gemm(L.qkvg, EPI_STORE, c->pf_big, c->nqkv, cut));
+            PCHK(gemm(L.qkvg, c->pf_big, c->nqkv, cut));
             pf_attn_args t{};
             t.qkv = c->pf_big;
             t.ld = c->nqkv;
@@ -139,7 +139,7 @@ int enqueue_chunk(sh_ctx* c, sh_state* st, int m, bool have_tokens, bool have_em
             t.cut = cut;
             PCHK(launch_pf_kv(t, s));
             PCHK(launch_pf_attn(t, s));
-            PCHK(gemm(L.o, EPI_STORE, c->pf_y, E, cut));
+            PCHK(gemm(L.o, c->pf_y, E, cut));
         }
         pf_rows_args f = r;
         f.conv = cv;
@@ -153,15 +153,8 @@ int enqueue_chunk(sh_ctx* c, sh_state* st, int m, bool have_tokens, bool have_em
         gu.in = cut;
         gu.out_ld = I.n_ff;
         gu.outc = act_cut;
-        if (pf_swiglu_cut_takes(gu)) {   // SwiGLU and the cut in the products' epilogue
-            PCHK(launch_pf_gemm(EPI_SWIGLU, gu, s));
-            PCHK(gemm(L.down, EPI_STORE, c->pf_y, E, act_cut));
-        } else {
-            PCHK(gemm(L.gate_up, EPI_SWIGLU, c->pf_act, I.n_ff, cut));
-            pf_cutk_args ck{c->pf_act, I.n_ff, I.n_ff, m, cut};
-            PCHK(launch_pf_cut(ck, s));
-            PCHK(gemm(L.down, EPI_STORE, c->pf_y, E, cut));
-        }
+        PCHK(launch_pf_gemm(EPI_SWIGLU, gu, s));   // SwiGLU and the cut in the products' epilogue
+        PCHK(gemm(L.down, c->pf_y, E, act_cut));
         pf_rows_args z = r;
         z.y = c->pf_y;
         z.w_post = L.post_ffn_norm;
