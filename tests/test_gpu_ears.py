@@ -47,6 +47,33 @@ def test_odd_table_sizes_match_oracle(model_dir, n):
     assert oracle.rel(out, ref) < TOL, oracle.rel(out, ref)
 
 
+# rows and columns that end inside a table tile; the wide ones' clips give position tiles that a wave's 2 or 4 do not divide
+SMALL = dict(n_mel=24, n_ch=8, n_embd=96, n_ff=40, n_head=3, n_head_kv=1, head_dim=32, layers="ca", window=5, n_out=264)
+WIDE = dict(n_mel=128, n_ch=136, n_embd=96, n_ff=2056, n_head=32, n_head_kv=1, head_dim=128, layers="ca", window=5, n_out=264)
+NORM = dict(n_mel=24, n_ch=8, n_embd=768, n_ff=40, n_head=3, n_head_kv=1, head_dim=32, layers="c", window=5, n_out=264)
+
+
+@pytest.mark.parametrize("kw,n", [(SMALL, 300), (SMALL, 5 * 16000 + 7), (WIDE, 384400), (NORM, 37123)],
+                         ids=["small-1", "small", "wide", "norm768"])
+def test_tables_bit_for_bit(model_dir, monkeypatch, kw, n):
+    """The rows equal the oracle's bit for bit where erff cannot make a difference: with a projector bias of 50 every
+    GELU input is far past the point from which erff is 1 in either library, so GELU is the identity in both."""
+    import nunchi_amd
+    from nunchi_amd import synth
+    add = synth.GGUFWriter.add_tensor
+
+    def biased(self, name, ty, dims, data):
+        return add(self, name, ty, dims, np.full_like(data, 50.0) if name == "mm.a.mlp.1.bias" else data)
+    monkeypatch.setattr(synth.GGUFWriter, "add_tensor", biased)
+    path = synth.write_ears(f"{model_dir}/ears_bits_{kw['n_embd']}_{kw['n_ff']}.gguf", synth.EarsShape(**kw), 4)
+    g = nunchi_amd.Ears(path)
+    out = g.encode(synth.clip(n, 8))
+    ref, mel = oracle.Ears(path, threads=8).encode(synth.clip(n, 8), mel=True)
+    assert np.array_equal(g.mel().view(np.uint32), mel.view(np.uint32))
+    assert out.shape == ref.shape
+    assert np.array_equal(out.view(np.uint32), ref.view(np.uint32)), oracle.rel(out, ref)
+
+
 def test_encode_repeats_and_shrinks(tiny_ears):
     """A longer clip, a shorter one (the work buffers are kept), then the first again: bit for bit the same rows."""
     import nunchi_amd
@@ -59,15 +86,17 @@ def test_encode_repeats_and_shrinks(tiny_ears):
     assert np.array_equal(rb.view(np.uint32), g.encode(b).view(np.uint32))
 
 
-def test_full_ears_hearing_window(model_dir):
-    """The full ears shape on a 30.7 s clip: the 384 rows of the hearing window."""
+@pytest.mark.parametrize("n,rows", [(37123, 29), (384400, 301), (491760, 384)])
+def test_full_ears(model_dir, n, rows):
+    """The full ears shape on a short clip, on one whose position tiles leave a remainder in the waves of the pointwise and
+    gate|up tables (1202 tiles by 4, 301 and 19 by 2), and on the 30.7 s of the hearing window."""
     import nunchi_amd
     from nunchi_amd import synth
     path = synth.cached("ears", synth.EARS, 3, model_dir)
-    pcm = synth.clip(491760, 1)
+    pcm = synth.clip(n, 1)
     out = nunchi_amd.Ears(path).encode(pcm)
     ref = oracle.Ears(path, threads=8).encode(pcm)
-    assert out.shape == ref.shape == (384, 2048)
+    assert out.shape == ref.shape == (rows, 2048)
     assert oracle.rel(out, ref) < TOL, oracle.rel(out, ref)
 
 

@@ -170,6 +170,25 @@ def test_prefill_partial_last_chunk(model_dir):
     assert same(lg, lp)
 
 
+@pytest.mark.parametrize("layer_type", ["q4_0", "q4_1"])
+@pytest.mark.parametrize("E,ff,n", [(288, 544, 45), (1376, 2080, 512)])
+def test_prefill_partial_last_chunk_types(model_dir, layer_type, E, ff, n):
+    """Tables of 9, 17, 43 and 65 blocks of either type against single steps, at sizes that take the narrow wave tile
+    (n 45) and the wide one (n 512: 4128 conv and 4160 gate|up rows)."""
+    import nunchi_amd
+    from nunchi_amd import synth
+    shape = synth.BrainShape(n_embd=E, n_layer=2, attn_layers=(1,), n_head=8, n_head_kv=4, head_dim=32, n_ff=ff,
+                             n_vocab=1000, layer_type=layer_type)
+    g = nunchi_amd.Brain(synth.cached("brain", shape, 28, model_dir), n_ctx=n + 1)
+    toks = _prompt(n, 1000, 29)
+    _, lg, _, ha = g.step_batch(toks, want_logits=True, hidden_all=True)
+    s = g.new_state()
+    for p, tok in enumerate(toks):
+        hp, lp, _ = g.step(int(tok), want_logits=p == n - 1, st=s)
+        assert same(hp, ha[p]), f"position {p}: batch and single step differ"
+    assert same(lg, lp)
+
+
 def test_prefill_attention_valu_form(tiny_model, monkeypatch):
     """The VALU attention (SEOUL_HIP_PF_ATTN_VALU=1, read per launch) gives the same numbers as the oracle too."""
     monkeypatch.setenv("SEOUL_HIP_PF_ATTN_VALU", "1")
