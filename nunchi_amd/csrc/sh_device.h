@@ -217,6 +217,48 @@ __device__ __forceinline__ float rms_scale_wave_g(Ptr x, float eps) {
     return 1.0f / sqrtf(s / (float)n + eps);
 }
 
+// the half-wave's chains over values [32 t, 32 (t + NT)) of R rows in memory, every operand requested first
+template <int R, int NT>
+__device__ __forceinline__ void half_chains(const float* const (&x)[R], int t, float (&a)[R]) {
+    const int hl = threadIdx.x & 31;
+    float v[R][NT];
+#pragma unroll
+    for (int q = 0; q < NT; q++)
+#pragma unroll
+        for (int i = 0; i < R; i++) v[i][q] = x[i][32 * (t + q) + hl];
+#pragma unroll
+    for (int q = 0; q < NT; q++)
+#pragma unroll
+        for (int i = 0; i < R; i++) a[i] = fmaf(v[i][q], v[i][q], a[i]);
+}
+
+// rms_scale_wave's values by a half-wave (lane P of the half runs chain P; the same combine) for R rows of n floats in
+// memory (n % 32 == 0), in every lane of the half. Bound by memory round trips: NT = n / 32 known when the kernel is
+// compiled takes one (R NT below 64: more requests fill a wave's load counter), NT = 0 (any width) one per 256 values and
+// one for each 32 past them
+template <int R, int NT>
+__device__ __forceinline__ void rms_scale_half(const float* const (&x)[R], int n, float eps, float (&out)[R]) {
+    static_assert(R * NT < 64, "requests in flight");
+    const int hl = threadIdx.x & 31, base = threadIdx.x & 32, nt = n / 32;
+    float a[R] = {};
+    if (NT > 0) {
+        half_chains<R, NT>(x, 0, a);
+    } else {
+        int t = 0;
+        for (; t + 8 <= nt; t += 8) half_chains<R, 8>(x, t, a);
+        for (; t < nt; t++) half_chains<R, 1>(x, t, a);
+    }
+    auto at = [&](float f, int l) { return __shfl(f, base + (l & 31)); };
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        const float u = (a[i] + at(a[i], hl + 8)) + (at(a[i], hl + 16) + at(a[i], hl + 24));   // lanes 0..7 of the half
+        const float r = u + at(u, hl + 4);
+        const float q = r + at(r, hl + 2);
+        const float s = at(q, 0) + at(q, 1);
+        out[i] = 1.0f / sqrtf(s / (float)n + eps);
+    }
+}
+
 // q or k of one head: norm (imi's order) times its weight, then the NEOX rope with the host's cos/sin row of this
 // position (imi/core/seoul.cpp:19-28). One wave; lane holds dimensions lane + 64 c (c < DPL), so at D 128 a rope pair
 // (i, i + 64) sits in one lane and at D <= 64 the partner comes by a shuffle. stg: D floats of staging.

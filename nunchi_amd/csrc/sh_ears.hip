@@ -13,58 +13,6 @@ constexpr int ET = 256;
 
 __device__ __forceinline__ float gelu_erf(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
-// imi_rms_scale (imi/core/vec.h:20-33) in its AVX2 op order by one half-wave over one row of n floats (n % 32 == 0):
-// lane P of the half runs the fma chain of x[32t + P]^2 over t (all loads issued first, 8 at a time), then
-// v_l = (a_l + a_{l+8}) + (a_{l+16} + a_{l+24}) and ((v0+v4) + (v2+v6)) + ((v1+v5) + (v3+v7)); every lane of the
-// half gets 1 / sqrtf(s / n + eps)
-__device__ __forceinline__ float rms_scale_half(const float* x, int n, float eps) {
-    const int lane = threadIdx.x & 63, hl = lane & 31, base = lane & 32;
-    const int nt = n / 32;
-    float a = 0.0f;
-    int t = 0;
-    for (; t + 8 <= nt; t += 8) {
-        float v[8];
-#pragma unroll
-        for (int q = 0; q < 8; q++) v[q] = x[32 * (t + q) + hl];
-#pragma unroll
-        for (int q = 0; q < 8; q++) a = fmaf(v[q], v[q], a);
-    }
-    for (; t < nt; t++) a = fmaf(x[32 * t + hl], x[32 * t + hl], a);
-    auto at = [&](float v, int l) { return __shfl(v, base + (l & 31)); };
-    const float v = (a + at(a, hl + 8)) + (at(a, hl + 16) + at(a, hl + 24));   // lanes 0..7 of the half
-    const float r = v + at(v, hl + 4);
-    const float q = r + at(r, hl + 2);
-    const float s = at(q, 0) + at(q, 1);
-    return 1.0f / sqrtf(s / (float)n + eps);
-}
-
-
-// the same for two rows of 32 NT values, every operand of both requested before the chains start (one memory round trip)
-template <int NT>
-__device__ __forceinline__ void rms_scale_half2(const float* x0, const float* x1, float eps, float (&out)[2]) {
-    const int lane = threadIdx.x & 63, hl = lane & 31, base = lane & 32;
-    float v[2][NT], a[2] = {0.0f, 0.0f};
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        v[0][t] = x0[32 * t + hl];
-        v[1][t] = x1[32 * t + hl];
-    }
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        a[0] = fmaf(v[0][t], v[0][t], a[0]);
-        a[1] = fmaf(v[1][t], v[1][t], a[1]);
-    }
-    auto at = [&](float f, int l) { return __shfl(f, base + (l & 31)); };
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        const float u = (a[i] + at(a[i], hl + 8)) + (at(a[i], hl + 16) + at(a[i], hl + 24));   // lanes 0..7 of the half
-        const float r = u + at(u, hl + 4);
-        const float q = r + at(r, hl + 2);
-        const float s = at(q, 0) + at(q, 1);
-        out[i] = 1.0f / sqrtf(s / (float)(32 * NT) + eps);
-    }
-}
-
 // where feature e of position p sits in a table's input (sh_ears.h)
 __device__ __forceinline__ size_t xat(int e, int p, int ldx) {
     return ((((size_t)(e >> 5) * (ldx >> 4) + (p >> 4)) * 2 + ((e >> 4) & 1)) * 64 + (e & 3) * 16 + (p & 15)) * 4 + ((e >> 2) & 3);
@@ -324,8 +272,9 @@ __global__ __launch_bounds__(ET) void k_eflat(const float* a, int lda, int K, in
 
 // a workgroup is 16 positions x 64 features: each wave forms 4 positions' scales in imi's order (every workgroup of a
 // position forms the same scale), then h is written as a table input, a thread the four features of one 16-byte
-// word. Bound by memory round trips: every operand is requested before the chains at the ears' 768 width (5.4 -> 4.9 us a
-// launch at 384 positions, 5.0 -> 4.1 at 29)
+// word. Bound by memory round trips: a width of 256, 512 or 768 (NT = E / 32; 0 takes any) has every operand requested
+// before the chains (768: 5.4 -> 4.9 us a launch at 384 positions, 5.0 -> 4.1 at 29)
+template <int NT>
 __global__ __launch_bounds__(ET) void k_enorm(const float* x, const float* w, int E, int P, int ldh, float eps, float* h) {
     __shared__ float sc[16];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, p0 = blockIdx.x * 16, e0 = blockIdx.y * 64;
@@ -341,12 +290,7 @@ __global__ __launch_bounds__(ET) void k_enorm(const float* x, const float* w, in
     const float* r0 = x + (size_t)min(p0 + pq, P - 1) * E;
     const float* r1 = x + (size_t)min(p0 + pq + 2, P - 1) * E;
     float sq[2];
-    if (E == 768) {
-        rms_scale_half2<24>(r0, r1, eps, sq);
-    } else {
-        sq[0] = rms_scale_half(r0, E, eps);
-        sq[1] = rms_scale_half(r1, E, eps);
-    }
+    rms_scale_half<2, NT>({r0, r1}, E, eps, sq);
     if ((lane & 31) == 0) {
         sc[pq] = sq[0];
         sc[pq + 2] = sq[1];
@@ -544,7 +488,13 @@ hipError_t launch_eflat(const float* a, int lda, int C, int F8, int P, float* xf
 hipError_t launch_enorm(const float* x, const float* w, int E, int P, float eps, float* h, int ldh, hipStream_t s) {
     if (E % 32) return hipErrorInvalidValue;
     if (ldh % 16) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_enorm, dim3((unsigned)(ldh / 16), (unsigned)((E + 63) / 64)), dim3(ET), 0, s, x, w, E, P, ldh, eps, h);
+    const dim3 grid((unsigned)(ldh / 16), (unsigned)((E + 63) / 64));
+    switch (E) {
+        case 256: hipLaunchKernelGGL((k_enorm<8>), grid, dim3(ET), 0, s, x, w, E, P, ldh, eps, h); break;
+        case 512: hipLaunchKernelGGL((k_enorm<16>), grid, dim3(ET), 0, s, x, w, E, P, ldh, eps, h); break;
+        case 768: hipLaunchKernelGGL((k_enorm<24>), grid, dim3(ET), 0, s, x, w, E, P, ldh, eps, h); break;
+        default: hipLaunchKernelGGL((k_enorm<0>), grid, dim3(ET), 0, s, x, w, E, P, ldh, eps, h);
+    }
     return hipGetLastError();
 }
 hipError_t launch_econv(const float* big, int ld, const float* w, int E, int d_conv, int P, float* act, int lda,

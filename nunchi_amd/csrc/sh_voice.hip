@@ -28,35 +28,21 @@ __device__ __forceinline__ void position_scales(const vtab_args& a, float* scl) 
     }
 }
 
-// rms_scale_wave's values by a half-wave (lane P of the half runs chain P; the same combine) over a row of 32 NT values in
-// memory, every operand requested first; in every lane of the half
-template <int NT>
-__device__ __forceinline__ float rms_scale_half_g(const float* x, float eps) {
-    const int hl = threadIdx.x & 31, base = threadIdx.x & 32;
-    float v[NT], a = 0.0f;
-#pragma unroll
-    for (int t = 0; t < NT; t++) v[t] = x[32 * t + hl];
-#pragma unroll
-    for (int t = 0; t < NT; t++) a = fmaf(v[t], v[t], a);
-    auto at = [&](float f, int l) { return __shfl(f, base + (l & 31)); };
-    const float u = (a + at(a, hl + 8)) + (at(a, hl + 16) + at(a, hl + 24));   // lanes 0..7 of the half
-    const float r = u + at(u, hl + 4);
-    const float q = r + at(r, hl + 2);
-    const float s = at(q, 0) + at(q, 1);
-    return 1.0f / sqrtf(s / (float)(32 * NT) + eps);
-}
-
-// position_scales with a half-wave per row for the widths the scaled-order tables have (the four waves' eight rows at once)
+// position_scales with a half-wave per row (the four waves' eight rows at once), in one round trip where the width is a multiple
+// of 256 up to 1024
 template <int P>
 __device__ __forceinline__ void position_scales_half(const vtab_args& a, float* scl) {
-    if (a.W.cols != 512 && a.W.cols != 1024) {
-        position_scales<P>(a, scl);
-        return;
-    }
     for (int p = threadIdx.x >> 5; p < P; p += VX_THREADS / 32) {
-        const float* row = a.src + (size_t)p * a.src_ld;
-        const float s = a.W.cols == 512 ? rms_scale_half_g<16>(row, a.eps) : rms_scale_half_g<32>(row, a.eps);
-        if ((threadIdx.x & 31) == 0) scl[p] = s;
+        float s[1];
+        const float* const row[1] = {a.src + (size_t)p * a.src_ld};
+        switch (a.W.cols) {
+            case 256: rms_scale_half<1, 8>(row, 256, a.eps, s); break;
+            case 512: rms_scale_half<1, 16>(row, 512, a.eps, s); break;
+            case 768: rms_scale_half<1, 24>(row, 768, a.eps, s); break;
+            case 1024: rms_scale_half<1, 32>(row, 1024, a.eps, s); break;
+            default: rms_scale_half<1, 0>(row, a.W.cols, a.eps, s);
+        }
+        if ((threadIdx.x & 31) == 0) scl[p] = s[0];
     }
 }
 
