@@ -50,11 +50,12 @@ def test_odd_table_sizes_match_oracle(model_dir, n):
 # rows and columns that end inside a table tile; the wide ones' clips give position tiles that a wave's 2 or 4 do not divide
 SMALL = dict(n_mel=24, n_ch=8, n_embd=96, n_ff=40, n_head=3, n_head_kv=1, head_dim=32, layers="ca", window=5, n_out=264)
 WIDE = dict(n_mel=128, n_ch=136, n_embd=96, n_ff=2056, n_head=32, n_head_kv=1, head_dim=128, layers="ca", window=5, n_out=264)
-NORM = dict(n_mel=24, n_ch=8, n_embd=768, n_ff=40, n_head=3, n_head_kv=1, head_dim=32, layers="c", window=5, n_out=264)
+NORM = dict(n_mel=24, n_ch=8, n_ff=40, n_head=3, n_head_kv=1, head_dim=32, layers="c", window=5, n_out=264)
 
 
-@pytest.mark.parametrize("kw,n", [(SMALL, 300), (SMALL, 5 * 16000 + 7), (WIDE, 384400), (NORM, 37123)],
-                         ids=["small-1", "small", "wide", "norm768"])
+@pytest.mark.parametrize("kw,n", [(SMALL, 300), (SMALL, 5 * 16000 + 7), (WIDE, 384400)] +
+                         [(dict(NORM, n_embd=E), 37123) for E in (256, 512, 768, 800)],
+                         ids=["small-1", "small", "wide", "norm256", "norm512", "norm768", "norm800"])
 def test_tables_bit_for_bit(model_dir, monkeypatch, kw, n):
     """The rows equal the oracle's bit for bit where erff cannot make a difference: with a projector bias of 50 every
     GELU input is far past the point from which erff is 1 in either library, so GELU is the identity in both."""

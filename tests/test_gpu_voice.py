@@ -70,10 +70,11 @@ def test_codebook_counts(model_dir, n_cb, schedule):
     _play(path, n_cb, schedule, n_frames=1)
 
 
-@pytest.mark.parametrize("n_cb,E,n_ff", [(12, 288, 800), (6, 512, 288), (12, 1024, 2080), (6, 96, 32)])
+@pytest.mark.parametrize("n_cb,E,n_ff", [(12, 288, 800), (6, 512, 288), (12, 1024, 2080), (6, 96, 32), (6, 768, 96),
+                                          (12, 1568, 64)])
 def test_scaled_order_widths(model_dir, n_cb, E, n_ff):
     """The scaled order's tables at widths that end inside a 256-column chunk (and are narrower than one), and the norm
-    scales' half-wave widths (512 and 1024)."""
+    scales of one round trip (512, 768 and 1024 columns) and of several (1568: 6 batches and a rest)."""
     from nunchi_amd import synth
     path = synth.cached("voice", _shape(n_cb=n_cb, n_embd=E, n_ff=n_ff, n_layer=1, n_vocab=96), 10, model_dir)
     _play(path, n_cb + E, (n_cb // 2, n_cb // 2), n_frames=1)
