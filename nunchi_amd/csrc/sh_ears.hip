@@ -49,7 +49,8 @@ __device__ __forceinline__ float wval(const wraw<F32W>& r, int s) {   // (s know
 // The float tables on the matrix cores, in imi_wg_group12's order (imi/core/tables.cpp:522-556): one chain
 // acc = fma(w, x, acc) per row and position over the columns in order. v_mfma_f32_16x16x4_f32 runs four columns of 16
 // rows x 16 positions: its four K steps are four fused multiply-adds in order, each rounded once, bit for bit the VALU's
-// fmaf chain (measured over 3 M random cases of spread exponents). A chain then takes 8 cycles a column, the rate of one
+// fmaf chain (no mismatch in 11 M random chains: 3 M of spread exponents, 8 M with denormals, signed zeros and overflow; the
+// ears' bit-for-bit tests rest on it). A chain then takes 8 cycles a column, the rate of one
 // matrix core in fp32, with a single chain per wave in flight; v_mfma_f32_4x4x1_16b_f32, one column per instruction,
 // is as fast only with two waves to cover its 15-cycle dependency, and wants a weight conversion and an operand word per
 // lane for every 64 x 4 outputs and column, where this takes them for 16 x 16 outputs and four columns.
@@ -59,11 +60,13 @@ __device__ __forceinline__ float wval(const wraw<F32W>& r, int s) {   // (s know
 // load costs its wave about as many cycles as one of these products), requested DC chunks of 32 columns ahead. Every
 // global load is unconditional (chunk indices clamped; past the table's last column nothing is multiplied), so the
 // compiler's wait counts stay exact.
-// At 384 positions, against one column per v_mfma_f32_4x4x1_16b_f32: b|c|x 2304 x 768 33.0 -> 21.2 us, gate|up 4096 x 768
-// 44.7 -> 30.0, o and down (768 x 768, 768 x 2048) 33.7 -> 19.3 on average, mlp.3 2048 x 2048 63.6 -> 37.4, pre_encode
-// 768 x 4096 90.7 -> 47.3. (With this product but feature-major inputs, read a word per step: 28.0, 44.0, 33.4, 51.3 and
-// 65.3; at 29 positions gate|up 12.6 and down 24.6 against 9.4 and 16.6.) Bound by the vector loads (3 KB per 32 columns
-// and 16 x 16 outputs), then by the chains' 8 cycles a column.
+// At 384 positions, against one column per v_mfma_f32_4x4x1_16b_f32: b|c|x 2304 x 768 33.7 -> 21.2 us, gate|up 4096 x 768
+// 45.5 -> 30.1, o and pw2 768 x 768 20.3 -> 12.8, down 768 x 2048 47.7 -> 26.3, mlp.3 2048 x 2048 63.7 -> 37.8, pre_encode
+// 768 x 4096 91.7 -> 47.6; at 29 positions b|c|x 16.9 -> 8.8, gate|up 17.7 -> 9.7, down 39.3 -> 17.2, pre_encode 76.2 ->
+// 30.8. (With this product but feature-major inputs, read a word per step: b|c|x 28.0, gate|up 44.0, mlp.3 51.3, pre_encode
+// 65.3; at 29 positions gate|up 12.6.) The matrix cores are busy 14 % (o, pw2) to 48 % (mlp.3) of the time at 384
+// positions: a 768-row table has 1152 tiles for 1024 SIMDs, a wave's chain takes 8 cycles a column (2048 columns 6.8 us),
+// and its loads (3 KB per 32 columns and 16 x 16 outputs) are issued between the products.
 template <int EPI, bool F32W, int MP>
 __global__ __launch_bounds__(ET) void k_etab(etab_args a) {
     typedef float v4f __attribute__((ext_vector_type(4)));

@@ -151,7 +151,7 @@ int ensure_work(sh_ears* e, int n) {
               P8 = pad16((long)g.P * g.F8);
     std::vector<size_t> sz = {
         (size_t)n,                                        // pcm
-        (size_t)pad32(N_FFT) * Pf,                               // fx
+        (size_t)pad32(N_FFT) * Pf,                        // fx
         (size_t)N_BIN * Pf,                               // pw
         (size_t)g.n_fr * I.n_mel,                         // mel
         (size_t)C * g.T2 * g.F2,                          // a0
@@ -164,7 +164,7 @@ int ensure_work(sh_ears* e, int n) {
         (size_t)std::max(E, I.n_embd) * Pp,               // h
         (size_t)g.P * e->big_w,                           // big
         (size_t)pad32(std::max({I.n_ff, I.n_head * std::max(I.head_dim, 1), E})) * Pp,   // act
-        (size_t)pad32(e->n_mid) * Pp,                       // proj
+        (size_t)pad32(e->n_mid) * Pp,                     // proj
         (size_t)g.P * I.n_out,                            // out
         (size_t)g.P * std::max(I.head_dim, 2),            // cs (float2 [P][D / 2])
     };

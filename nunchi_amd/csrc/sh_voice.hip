@@ -28,8 +28,8 @@ __device__ __forceinline__ void position_scales(const vtab_args& a, float* scl) 
     }
 }
 
-// position_scales with a half-wave per row (the four waves' eight rows at once), in one round trip where the width is a multiple
-// of 256 up to 1024
+// position_scales with a half-wave per row (the four waves' eight rows at once), in one round trip where the width is a
+// multiple of 256 up to 1024
 template <int P>
 __device__ __forceinline__ void position_scales_half(const vtab_args& a, float* scl) {
     for (int p = threadIdx.x >> 5; p < P; p += VX_THREADS / 32) {
@@ -265,16 +265,19 @@ __global__ __launch_bounds__(VX_THREADS) void k_vtab_fold(vtab_args a) {
 // scaled order (imi/core/tables.cpp:324-365, P = 12 or 6): one chain per (row, position) over all columns of
 // fma(float(w) * d, x, acc); two row groups (16 rows) per workgroup, which are one 16 x 16 tile of
 // v_mfma_f32_16x16x4_f32 (positions past P repeat the last one and are dropped): its four K steps are four fused
-// multiply-adds in column order, each rounded once, bit for bit the VALU's chain, at 8 cycles a column where a dependent
-// VALU chain with its LDS reads ran at 15. A fifth wave runs the chains while the other four stage; its lane l supplies row / position l % 16, column l / 16 of
-// a step, and holds rows 4 (l / 16) + i of position l % 16. The workgroup stages 256 columns at a time, one chunk
-// ahead, requested one more chunk before that: each thread loads one 16-byte word of codes (16 columns of one row's block) and the block's scale and stores the
-// 16 products float(w) * d (exact: an int8 times an fp16 has at most 19 significant bits) to LDS, and the positions'
-// inputs (normed first for a VP_NORM table) beside them. Within each 16 columns LDS holds column 4 s + k at 4 k + s, so
-// a lane's four steps are one 16-byte word each.
-// Against a thread per chain: 512 columns 8.2 -> 6.0 us a launch (norm in front), 2048 columns 16 -> 13.3, 4096 at 12
-// positions 22.1; bound by the chains' dependent products (33 cycles a step) and, at 512 columns, by the launch, the norm's
-// own chain and the first chunk's way in.
+// multiply-adds in column order, each rounded once, bit for bit the VALU's chain (k_etab), at 8 cycles a column where a
+// dependent VALU chain with its LDS reads ran at 15. A fifth wave runs the chains while the other four stage; its lane l
+// supplies row / position l % 16, column l / 16 of a step, and holds rows 4 (l / 16) + i of position l % 16. The workgroup
+// stages 256 columns at a time, one chunk ahead, requested one more chunk before that: each thread loads one 16-byte word
+// of codes (16 columns of one row's block) and the block's scale and stores the 16 products float(w) * d (exact: an int8
+// times an fp16 has at most 19 significant bits) to LDS, and the positions' inputs (normed first for a VP_NORM table)
+// beside them. Within each 16 columns LDS holds column 4 s + k at 4 k + s, so a lane's four steps are one 16-byte word
+// each.
+// Against a thread per chain, us a launch: 6 positions, 512 columns 5.8 -> 4.9 (norm in front 8.2 -> 5.5, gate|up 8.8 ->
+// 6.0), 2048 columns 16.7 -> 12.2; 12 positions, 1024 columns 9.6 -> 7.5 (norm in front 13.2 -> 9.8; gate|up, two
+// workgroups a CU, 17.9 -> 18.6), 4096 columns 32.7 -> 22.1. A launch is 2.4 us and 19 ns per four columns: 46 cycles at 2.4 GHz, of
+// which the dependent product takes 33 and the chunks' barriers and first LDS reads the rest; a norm in front adds its
+// row's round trip and chain (0.6 to 2.3 us). Matrix cores and VALU are busy 1 to 6 % and 1 to 11 % of the time.
 template <int P, int PRO, int EPI>
 __global__ __launch_bounds__(VX_THREADS + 64) void k_vtab_scaled(vtab_args a) {
     const uint64_t et = EPI == VE_SWIGLU ? kExp2Tab[threadIdx.x & 31] : 0;   // (first: its wait needs nothing later)
